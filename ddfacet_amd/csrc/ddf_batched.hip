@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 #include <string>
@@ -432,21 +433,38 @@ __global__ void plan_block_desc(const VisP v, uint4* desc) {
 }
 
 __global__ void reset_counter(uint32_t* c, int n) {
-  if (threadIdx.x < n) c[threadIdx.x] = 0;
+  if (threadIdx.x < n) c[threadIdx.x * kQueueStride] = 0;
 }
 
-// Next work item of a tile pass for a workgroup, taken by one thread whose state (x, left) starts
-// at (blockIdx.x % n, n) for n item ranges.  Workgroups are dispatched to the 8 XCDs round robin,
-// so with 8 ranges the workgroups of one XCD take the items of their own range x (one counter per
-// range) in order; a workgroup whose range is used up moves on to the next ranges.  Returns
-// 0xFFFFFFFF once it has found every range used up (at most n failed atomics per workgroup).
-__device__ __forceinline__ uint32_t next_tile_item(uint32_t* queue, const uint32_t* range, int n, int& x,
-                                                   int& left) {
-  while (left > 0) {
-    const uint32_t it = range[x] + atomicAdd(queue + x, 1u);
-    if (it < range[x + 1]) return it;
-    x = x + 1 == n ? 0 : x + 1;
-    --left;
+// Next pack of work items of a tile pass for a workgroup, taken by one thread.  Workgroups are
+// dispatched to the 8 XCDs round robin, so with n = 8 ranges the workgroups of one XCD take the packs
+// of their own range x first (one counter per range) in order, and then what is left of the others.
+// A workgroup's first pack is that of its number in its range; the counters hand out those after.
+// Returns 0xFFFFFFFF once it has found every range used up.  (An atomic on one cache line is served
+// every 12 ns, whatever the counter in it, so the counters have a line each, and a range is only asked
+// where a plain load says that it may have packs: with 8 counters in a line and a failing atomic a
+// range and workgroup at the end, half a million items took 6.2 ms and a thousand 72 us.)
+struct PackQueue {
+  int x, left;
+  bool first;
+};
+__device__ __forceinline__ PackQueue pack_queue(int n) { return PackQueue{int(blockIdx.x % uint32_t(n)), n, true}; }
+__device__ __forceinline__ uint32_t next_tile_pack(uint32_t* queue, const uint32_t* range, int n, PackQueue& q) {
+  if (q.first) {
+    q.first = false;
+    const uint32_t at = range[q.x] + blockIdx.x / uint32_t(n);
+    if (at < range[q.x + 1]) return at;
+  }
+  while (q.left > 0) {
+    const uint32_t wgs = gridDim.x > uint32_t(q.x) ? (gridDim.x - uint32_t(q.x) + uint32_t(n) - 1) / uint32_t(n) : 0u;
+    const uint32_t begin = range[q.x] + wgs, end = range[q.x + 1];
+    uint32_t* c = queue + q.x * kQueueStride;
+    if (begin < end && __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < end - begin) {
+      const uint32_t at = atomicAdd(c, 1u);
+      if (at < end - begin) return begin + at;
+    }
+    q.x = q.x + 1 == n ? 0 : q.x + 1;
+    --q.left;
   }
   return 0xFFFFFFFFu;
 }
@@ -585,9 +603,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
     }
   };
 
-  while (true) {
+  for (bool first = true;; first = false) {
     if (threadIdx.x == 0) {
-      s_item = atomicAdd(queue, 1u);
+      s_item = first ? blockIdx.x : gridDim.x + atomicAdd(queue, 1u);
       s_next = 0;
     }
     __syncthreads();
@@ -1253,13 +1271,18 @@ __global__ __launch_bounds__(64) void grid_pass_b(BatchParams p, const uint64_t*
   const int WW = W * W;
   const int npg = ONE ? 1 : (p.nstokes < p.npol ? p.nstokes : p.npol);
   const int lane = threadIdx.x;
-  int qx = int(blockIdx.x % uint32_t(p.nranges)), qleft = p.nranges;
+  PackQueue q = pack_queue(p.nranges);
+  uint32_t it = 0, it1 = 0;  // the items left of the pack
   while (true) {
-    if (lane == 0) s_item = next_tile_item(queue, p.item_range, p.nranges, qx, qleft);
-    __syncthreads();
-    const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-    if (it >= p.nitems_b) break;
-    const BinItem bi = items[it];
+    if (it == it1) {
+      if (lane == 0) s_item = next_tile_pack(queue, p.pack_range, p.nranges, q);
+      __syncthreads();
+      const uint32_t pack = __builtin_amdgcn_readfirstlane(s_item);
+      if (pack >= p.npacks) break;
+      it = gptr(p.pack_first)[pack];
+      it1 = gptr(p.pack_first)[pack + 1];
+    }
+    const BinItem bi = items[it++];
     const FacetDev fd = gload(p.facets + bi.facet);
     // the CF base in scalar registers (the loads address it with a 32-bit vector offset)
     const uint64_t cfa = reinterpret_cast<uint64_t>(fd.cf);
@@ -1328,46 +1351,89 @@ __global__ __launch_bounds__(64) void grid_pass_b(BatchParams p, const uint64_t*
   }
 }
 
-// grid[f][band][pol][y][x] += the tile slots covering (y, x), one thread per grid cell: the
-// tiles ty with ty * T - h <= y < ty * T + T + h (at most two per axis when h < T), each with
-// its consecutive work items, in item order.  No atomics; the same sum order on every run.
+// grid[f][band][pol][y][x] += the tile slots covering (y, x): the tiles ty with ty * T - h <= y <
+// ty * T + T + h (at most two per axis when h < T), each with its consecutive work items, in item
+// order.  No atomics; the same sum order on every run.  Workgroups take the T x T tiles that have a slot
+// in their reach (the plan's list), a lane per cell, so grids whose uv plane is mostly empty cost what
+// is in them: 121 facets x 4 bands of 975^2, 1.9 ms (3.7 with a lane for every cell of
+// every grid).  Bound: HBM (the slots are read once, the touched cells read and written).
 __global__ __launch_bounds__(256) void grid_slot_reduce(BatchParams p, const float2* slots, const uint32_t* tile_first,
-                                                        const uint32_t* tile_count) {
+                                                        const uint32_t* tile_count, const uint32_t* live) {
   const int T = p.tile, h = p.halo;
   const int W = T + 2 * h;
   const int WW = W * W;
   const int npg = p.nstokes < p.npol ? p.nstokes : p.npol;
-  const int64_t total = int64_t(p.nf) * p.nband * npg * p.ny * p.nx;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += int64_t(gridDim.x) * blockDim.x) {
-    int64_t r = i;
-    const int x = int(r % p.nx); r /= p.nx;
-    const int y = int(r % p.ny); r /= p.ny;
-    const int ip = int(r % npg); r /= npg;
-    const int band = int(r % p.nband); r /= p.nband;
-    const int f = int(r);
-    float re = 0.f, im = 0.f;
-    const int ty0 = max(0, (y - h) / T), ty1 = min(p.ntiles_y - 1, (y + h) / T);
-    const int tx0 = max(0, (x - h) / T), tx1 = min(p.ntiles_x - 1, (x + h) / T);
-    for (int ty = ty0; ty <= ty1; ++ty) {
-      const int ly = y - (ty * T - h);
-      for (int tx = tx0; tx <= tx1; ++tx) {
-        const int lx = x - (tx * T - h);
-        const int64_t tid = ((int64_t(f) * p.nband + band) * p.ntiles_y + ty) * p.ntiles_x + tx;
-        const uint32_t first = tile_first[tid], n = tile_count[tid];
-        const float2* t = slots + size_t(first) * npg * WW + size_t(ip) * WW + size_t(ly) * W + lx;
-        for (uint32_t k = 0; k < n; ++k, t += size_t(npg) * WW) {
-          const float2 v = *t;
-          re += v.x;
-          im += v.y;
+  const uint32_t n_live = gptr(live)[0];
+  const uint32_t per = uint32_t(p.ntiles_x) * uint32_t(p.ntiles_y);
+  for (uint32_t k = blockIdx.x; k < n_live; k += gridDim.x) {
+    const uint32_t tid0 = gptr(live)[1 + k];
+    const uint32_t fb = tid0 / per, r0 = tid0 - fb * per;
+    const int f = int(fb / uint32_t(p.nband)), band = int(fb - uint32_t(f) * uint32_t(p.nband));
+    const int yt = int(r0 / uint32_t(p.ntiles_x)) * T, xt = int(r0 % uint32_t(p.ntiles_x)) * T;
+    DDF_GLOBAL float2* g = gptr_w(reinterpret_cast<float2*>(gload(p.facets + f).grid)) + size_t(band) * p.npol * p.ny * p.nx;
+    for (int c = threadIdx.x; c < T * T * npg; c += blockDim.x) {
+      const int ip = c / (T * T), r = c - ip * (T * T);
+      const int y = yt + r / T, x = xt + r % T;
+      if (y >= p.ny || x >= p.nx) continue;
+      float re = 0.f, im = 0.f;
+      const int ty0 = max(0, (y - h) / T), ty1 = min(p.ntiles_y - 1, (y + h) / T);
+      const int tx0 = max(0, (x - h) / T), tx1 = min(p.ntiles_x - 1, (x + h) / T);
+      for (int ty = ty0; ty <= ty1; ++ty) {
+        const int ly = y - (ty * T - h);
+        for (int tx = tx0; tx <= tx1; ++tx) {
+          const int lx = x - (tx * T - h);
+          const size_t tid = size_t(fb) * per + size_t(ty) * p.ntiles_x + tx;
+          const uint32_t first = gptr(tile_first)[tid], n = gptr(tile_count)[tid];
+          const DDF_GLOBAL float2* t = gptr(slots) + (size_t(first) * npg * WW + size_t(ip) * WW + size_t(ly) * W + lx);
+          uint32_t i = 0;
+          for (; i + 4 <= n; i += 4, t += size_t(4) * npg * WW) {
+            float2 v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = ld2(t + size_t(q) * npg * WW);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              re += v[q].x;
+              im += v[q].y;
+            }
+          }
+          for (; i < n; ++i, t += size_t(npg) * WW) {
+            const float2 v = ld2(t);
+            re += v.x;
+            im += v.y;
+          }
         }
       }
+      if (re != 0.f || im != 0.f) {
+        DDF_GLOBAL float2* o = g + (size_t(ip) * p.ny + y) * p.nx + x;
+        const float2 v = ld2(o);
+        st2(o, make_float2(v.x + re, v.y + im));
+      }
     }
-    if (re != 0.f || im != 0.f) {
-      DDF_GLOBAL float2* g = gptr_w(reinterpret_cast<float2*>(gload(p.facets + f).grid)) +
-                             ((size_t(band) * p.npol + ip) * p.ny + y) * p.nx + x;
-      const float2 o = ld2(g);
-      st2(g, make_float2(o.x + re, o.y + im));
+  }
+}
+
+// The tiles within reach of a tile with slots (a tile's stamps reach h cells past it).
+__global__ __launch_bounds__(256) void plan_live_tiles(BatchParams p, const uint32_t* tile_count, int64_t ntile,
+                                                       uint32_t* live) {
+  const int d = (p.halo + p.tile - 1) / p.tile;
+  const int per = p.ntiles_x * p.ntiles_y;
+  for (int64_t i0 = int64_t(blockIdx.x) * blockDim.x; i0 < ntile; i0 += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t i = i0 + threadIdx.x;
+    bool on = false;
+    if (i < ntile) {
+      const int64_t fb = i / per;
+      const int r = int(i - fb * per), ty = r / p.ntiles_x, tx = r - ty * p.ntiles_x;
+      for (int y = max(0, ty - d); y <= min(p.ntiles_y - 1, ty + d) && !on; ++y)
+        for (int x = max(0, tx - d); x <= min(p.ntiles_x - 1, tx + d) && !on; ++x)
+          on = tile_count[fb * per + int64_t(y) * p.ntiles_x + x] != 0;
     }
+    const uint64_t mask = __ballot(on);
+    if (!mask) continue;
+    const int lane = threadIdx.x & 63, lead = __builtin_ctzll(mask);
+    uint32_t base = 0;
+    if (lane == lead) base = atomicAdd(live, uint32_t(__popcll(mask)));
+    base = uint32_t(__shfl(int(base), lead, 64));
+    if (on) live[1 + base + __popcll(mask & ((1ull << lane) - 1))] = uint32_t(i);
   }
 }
 
@@ -1392,13 +1458,18 @@ __global__ __launch_bounds__(256) void degrid_pass_a(BatchParams p, const uint64
   const int W = p.tile + 2 * p.halo;
   const int WW = W * W;
   const int ns = ONE ? 1 : p.nstokes;
-  int qx = int(blockIdx.x % uint32_t(p.nranges)), qleft = p.nranges;
+  PackQueue q = pack_queue(p.nranges);
+  uint32_t it = 0, it1 = 0;  // the items left of the pack
   while (true) {
-    if (threadIdx.x == 0) s_item = next_tile_item(queue, p.item_range, p.nranges, qx, qleft);
-    __syncthreads();
-    const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-    if (it >= p.nitems_b) break;
-    const BinItem bi = items[it];
+    if (it == it1) {
+      if (threadIdx.x == 0) s_item = next_tile_pack(queue, p.pack_range, p.nranges, q);
+      __syncthreads();
+      const uint32_t pack = __builtin_amdgcn_readfirstlane(s_item);
+      if (pack >= p.npacks) break;
+      it = gptr(p.pack_first)[pack];
+      it1 = gptr(p.pack_first)[pack + 1];
+    }
+    const BinItem bi = items[it++];
     const FacetDev fd = gload(p.facets + bi.facet);
     const DDF_GLOBAL float2* cfp = gptr(fd.cft);
     const int x0 = bi.tx * p.tile - p.halo, y0 = bi.ty * p.tile - p.halo;
@@ -1786,8 +1857,8 @@ __global__ __launch_bounds__(256) void degrid_adj_b(BatchParams p, const VisP v,
   const int lf = threadIdx.x - slot * G;
   const bool active = slot < slots;
   __shared__ uint32_t s_item;
-  while (true) {
-    if (threadIdx.x == 0) s_item = atomicAdd(queue, 1u);
+  for (bool first = true;; first = false) {
+    if (threadIdx.x == 0) s_item = first ? blockIdx.x : gridDim.x + atomicAdd(queue, 1u);
     __syncthreads();
     const uint32_t item = s_item;
     if (item >= p.nitems_a) break;
@@ -2022,6 +2093,7 @@ int batched_grid_a(const BatchParams& p, const VisP& v, const uint8_t* pcode, fl
                    unsigned nwg, hipStream_t st) {
   size_t lds = (size_t(p.nf) * (p.nband * p.npol + 2 * p.nband) + (p.chan_lds ? size_t(p.group) * (2 * v.nchan + 1) : 0)) * 8 +
                batched_grid_a_stage_bytes(p.group, p.read);
+  nwg = std::min(nwg, p.nitems_a);
   if (p.read == 4) launch_a_j<4>(p, v, pcode, V, queue, lds, nwg, st);
   else if (p.read == 2) launch_a_j<2>(p, v, pcode, V, queue, lds, nwg, st);
   else launch_a_j<1>(p, v, pcode, V, queue, lds, nwg, st);
@@ -2075,7 +2147,7 @@ int batched_tile_wgs(const BatchParams& pg, const BatchParams& pd, unsigned out[
   const int npd = pd.nstokes < pd.npol ? pd.nstokes : pd.npol;
   out[0] = persistent_wgs(grid_pass_b_for<false, false>(npg, pg.halo), grid_pass_b_lds(npg, Wg, false), 0, 64);
   const size_t lds_d = size_t(pd.nstokes) * Wd * Wd * 2 * sizeof(float);
-  out[1] = persistent_wgs(degrid_pass_a_for(pd.prec, pd.nstokes == 1), lds_d, 0);
+  out[1] = persistent_wgs(degrid_pass_a_for(pd.prec, pd.nstokes == 1), lds_d, 0, pd.tile_threads);
   out[2] = persistent_wgs(grid_pass_b_adjoint_for(npd, pd.halo, Wd, pd.prec),
                           grid_pass_b_lds(npd, Wd, adjoint_wide(npd, Wd, pd.prec)), 0, 64);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
@@ -2083,21 +2155,29 @@ int batched_tile_wgs(const BatchParams& pg, const BatchParams& pd, unsigned out[
 
 int batched_grid_b(const BatchParams& p, const uint64_t* place, const float2* V, const BinItem* items,
                    const uint32_t* recs, uint32_t* queue, unsigned nwg, float* slots, const uint32_t* tile_first,
-                   const uint32_t* tile_count, hipStream_t st) {
+                   const uint32_t* tile_count, const uint32_t* live, hipStream_t st) {
   const int W = p.tile + 2 * p.halo;
   const int npg = p.nstokes < p.npol ? p.nstokes : p.npol;
   const size_t lds = grid_pass_b_lds(npg, W, false);
+  nwg = std::min(nwg, p.npacks);
   hipLaunchKernelGGL((grid_pass_b_for<false, false>(npg, p.halo)), dim3(nwg), dim3(64), lds, st, p, place, V, items, recs,
                      queue, reinterpret_cast<float2*>(slots));
   if (hipGetLastError() != hipSuccess) return DDF_EHIP;
   if (slots) {
-    const int64_t total = int64_t(p.nf) * p.nband * npg * p.ny * p.nx;
-    int64_t nb = (total + 255) / 256;
-    if (nb > 8192) nb = 8192;
-    if (nb < 1) nb = 1;
+    int64_t nb = int64_t(p.nf) * p.nband * p.ntiles_y * p.ntiles_x;
+    if (nb > 4096) nb = 4096;
     hipLaunchKernelGGL(grid_slot_reduce, dim3(unsigned(nb)), dim3(256), 0, st, p, reinterpret_cast<const float2*>(slots),
-                       tile_first, tile_count);
+                       tile_first, tile_count, live);
   }
+  return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
+}
+
+int batched_live_tiles(const BatchParams& p, const uint32_t* tile_count, uint32_t* live, hipStream_t st) {
+  const int64_t ntile = int64_t(p.nf) * p.nband * p.ntiles_y * p.ntiles_x;
+  int64_t nb = (ntile + 255) / 256;
+  if (nb > 65536) nb = 65536;
+  if (batched_reset(live, 1, st)) return DDF_EHIP;
+  hipLaunchKernelGGL(plan_live_tiles, dim3(unsigned(nb)), dim3(256), 0, st, p, tile_count, ntile, live);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
 }
 
@@ -2109,6 +2189,7 @@ int batched_degrid_a_adjoint(const BatchParams& p, const uint64_t* place, const 
   q.npol = p.npol;
   const int npg = q.nstokes < q.npol ? q.nstokes : q.npol;
   const size_t lds = grid_pass_b_lds(npg, W, adjoint_wide(npg, W, q.prec));
+  nwg = std::min(nwg, p.npacks);
   hipLaunchKernelGGL(grid_pass_b_adjoint_for(npg, q.halo, W, q.prec), dim3(nwg), dim3(64), lds, st, q, place, Mbar, items, recs,
                      queue, static_cast<float2*>(nullptr));
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
@@ -2119,8 +2200,7 @@ int batched_degrid_a(const BatchParams& p, const uint64_t* place, float2* M, con
   const int W = p.tile + 2 * p.halo;
   const size_t lds = size_t(p.nstokes) * W * W * 2 * sizeof(float);
   const DegridPassA k = degrid_pass_a_for(p.prec, p.nstokes == 1);
-  nwg = persistent_wgs(k, lds, nwg);
-  hipLaunchKernelGGL(k, dim3(nwg), dim3(256), lds, st, p, place, M, items, recs, queue);
+  hipLaunchKernelGGL(k, dim3(std::min(nwg, p.npacks)), dim3(p.tile_threads), lds, st, p, place, M, items, recs, queue);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
 }
 
@@ -2191,6 +2271,7 @@ static void launch_adj_b_j(const BatchParams& p, const VisP& v, const uint8_t* p
 
 int batched_degrid_b_adjoint(const BatchParams& p, const VisP& v, const uint8_t* pcode, const float2* vbar,
                              float2* Mbar, uint32_t* queue, unsigned nwg, hipStream_t st) {
+  nwg = std::min(nwg, p.nitems_a);
   if (v.ncorr == 4) launch_adj_b_j<4>(p, v, pcode, vbar, Mbar, queue, nwg, st);
   else if (v.ncorr == 2) launch_adj_b_j<2>(p, v, pcode, vbar, Mbar, queue, nwg, st);
   else launch_adj_b_j<1>(p, v, pcode, vbar, Mbar, queue, nwg, st);

@@ -165,10 +165,18 @@ struct FacetDev {
   double* sum_jones_chan;  // [2][nchan]
 };
 
+// Words between two queue counters (a cache line each).
+constexpr int kQueueStride = 32;
 // Work-item ranges of a tile pass, one per XCD (workgroup b is dispatched to XCD b % 8), for plans
 // of at least kRangeMinItems work items.
 constexpr int kItemRanges = 8;
 constexpr size_t kRangeMinItems = 65536;
+
+// A pack closes at kPackRecords records or at kPackItems items (fewer where the plan has few items).
+constexpr uint32_t kPackRecords = 512, kPackItems = 16;
+// A tile of at most this many records is one item whatever its CF planes (four groups of planes
+// otherwise, see build_bins).
+constexpr int64_t kWholeTileRecords = 512;
 
 struct BinItem {
   uint32_t begin, end;     // record range in the binned record list
@@ -204,10 +212,14 @@ struct BatchParams {
   // tiles
   int tile, halo, ntiles_x, ntiles_y;
   uint32_t nitems_b;
-  // the work items split into nranges (1 or kItemRanges) contiguous ranges of about equal record
-  // counts: range x is items [item_range[x], item_range[x + 1])
-  const uint32_t* item_range;
+  // consecutive work items are queued in packs: pack k is items [pack_first[k], pack_first[k + 1]).
+  uint32_t npacks;
+  const uint32_t* pack_first;
+  // the packs split into nranges (1 or kItemRanges) contiguous ranges of about equal record counts:
+  // range x is packs [pack_range[x], pack_range[x + 1])
+  const uint32_t* pack_range;
   int nranges;
+  int tile_threads;  // workgroup of degrid pass A
   // blocks of the pass's BDA map: the per-(block, facet) values between the passes are stored
   // facet-major, [facet][block][nstokes]
   int64_t nblk;
@@ -243,7 +255,9 @@ int batched_grid_a(const BatchParams& p, const VisP& v, const uint8_t* pcode, fl
 // ([nitems][npg][2][W*W]) and grid_slot_reduce (tile_first / tile_count: the items of each tile)
 int batched_grid_b(const BatchParams& p, const uint64_t* place, const float2* V, const BinItem* items,
                    const uint32_t* recs, uint32_t* queue, unsigned nwg, float* slots, const uint32_t* tile_first,
-                   const uint32_t* tile_count, hipStream_t st);
+                   const uint32_t* tile_count, const uint32_t* live, hipStream_t st);
+// live[0]: how many tiles of a (facet, band) have slots in their reach, live[1 ...] which (any order)
+int batched_live_tiles(const BatchParams& p, const uint32_t* tile_count, uint32_t* live, hipStream_t st);
 int batched_degrid_a(const BatchParams& p, const uint64_t* place, float2* M, const BinItem* items,
                      const uint32_t* recs, uint32_t* queue, unsigned nwg, hipStream_t st);
 // vrun / run_first: the runs of the degrid visibility list (batched_run_ids)

@@ -1281,6 +1281,7 @@ struct ddf_plan {
   float* slots_g = nullptr;      // one LDS tile image per grid work item (null: atomic flush)
   uint32_t* tile_first_g = nullptr;
   uint32_t* tile_count_g = nullptr;
+  uint32_t* live_g = nullptr;    // count, then the tiles that have slots in reach
   uint64_t* bstamp_d = nullptr;
   BinItem* items_g = nullptr;
   BinItem* items_d = nullptr;
@@ -1292,9 +1293,11 @@ struct ddf_plan {
   uint32_t* vrun = nullptr;       // run of each degrid list entry (block and Jones key shared)
   uint32_t* run_first = nullptr;  // first list entry of each run
   int64_t nruns = 0;
-  // work-queue counters: [0] grid pass A, [1, 9) grid pass B (one per item range), [9, 17) degrid
+  // work-queue counters (kQueueStride words apart): [0] grid pass A, [1, 9) grid pass B (one per item range), [9, 17) degrid
   // pass A, [17] the adjoint of degrid pass B, [18, 26) the adjoint of degrid pass A
+  static constexpr int kQueues = 2 + 3 * kItemRanges;
   uint32_t* queues = nullptr;
+  uint32_t* queue(int k) const { return queues + k * kQueueStride; }
   const float2* jsrc[2] = {nullptr, nullptr};  // caller's DD / beam Jones tables
   double2* jprep[2] = {nullptr, nullptr};      // prepared copies (JonesP::pk / pb)
   float2* jprepf[2] = {nullptr, nullptr};      // complex64 prepared copies (JonesP::pkf / pbf)
@@ -1423,8 +1426,7 @@ void fill_batch(BatchParams& p, const ddf_grid_desc* g, const ddf_facet* f0, con
 
 // Count -> scan -> fill of the valid records, then the work items (largest first).
 int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place, int chunk, uint32_t** recs_out,
-               BinItem** items_out, uint32_t* nitems, int64_t* nrec, const uint32_t** ranges_out, int* nranges_out,
-               bool stamp_order,
+               BinItem** items_out, uint32_t* nitems, int64_t* nrec, bool stamp_order,
                hipStream_t st, uint32_t** tile_first_out = nullptr, uint32_t** tile_count_out = nullptr) {
   const int64_t nsub = 2 * int64_t(p.nw);  // CF-plane sub-bins of each tile
   const int64_t ntile_all = int64_t(p.nf) * p.nband * p.ntiles_y * p.ntiles_x;
@@ -1449,6 +1451,25 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
   std::vector<uint32_t> hg(static_cast<size_t>(ntile_all * ngrp));
   HIP_TRY(hipMemcpyAsync(hg.data(), gcount, hg.size() * 4, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
+  // Records of an item: those asked for, or 2048, down to 64 where a plan has too few to give every
+  // wavefront of the tile passes an item (9 facets of 189^2, 11 000 records: a wavefront with a heavy
+  // tile's 1000 records took longer than all others together).
+  if (chunk <= 0) {
+    int64_t all = 0;
+    for (uint32_t c : hg) all += c;
+    chunk = int(std::min<int64_t>(2048, std::max<int64_t>(64, all / 4096 / 64 * 64)));
+  }
+  // A light tile is one item: its groups' counts go to the first group (121 facets x 4 bands: 506 000
+  // items of 37 records otherwise, each with a tile to clear and a slot to write).
+  const int64_t whole = std::min<int64_t>(chunk, kWholeTileRecords);
+  for (int64_t i = 0; i < ntile_all; ++i) {
+    uint32_t* h = &hg[size_t(i * ngrp)];
+    int64_t all = 0;
+    for (int64_t g = 0; g < ngrp; ++g) all += h[g];
+    if (all > whole) continue;
+    std::fill(h, h + ngrp, 0u);
+    h[0] = uint32_t(all);
+  }
   // tile-major pass: each tile's first record and first slot, each (tile, group)'s item count
   std::vector<int64_t> ts(static_cast<size_t>(ntile_all));
   std::vector<uint32_t> tfirst(static_cast<size_t>(ntile_all)), tcount(static_cast<size_t>(ntile_all));
@@ -1496,31 +1517,48 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
   HIP_TRY(hipMemcpyAsync(tstart, ts.data(), ts.size() * 8, hipMemcpyHostToDevice, st));
   if (batched_bin_starts(counts, tstart, ntile_all, int(nsub), bstart, st))
     return fail(DDF_EHIP, "plan_bin_starts launch failed");
+  // packs of consecutive items
+  const size_t pack_items = std::min<size_t>(kPackItems, std::max<size_t>(1, items.size() / 16384));
+  std::vector<uint32_t> packs;
+  packs.reserve(items.size() / pack_items + 2);
+  for (size_t k = 0; k < items.size();) {
+    packs.push_back(uint32_t(k));
+    uint32_t n = 0;
+    for (size_t k0 = k; k < items.size() && k - k0 < pack_items && n < kPackRecords; ++k) n += items[k].end - items[k].begin;
+  }
+  const uint32_t npacks = uint32_t(packs.size());
+  packs.push_back(uint32_t(items.size()));
   // kItemRanges contiguous ranges of the launch order with about equal record counts: the
-  // workgroups of one XCD take the items of their own range first, so the items in flight on an
+  // workgroups of one XCD take the packs of their own range first, so the items in flight on an
   // XCD come from few (facet, plane group)s and their CF planes stay in that XCD's L2.  Only with
   // many items: with few, the heaviest items (neighbouring uv tiles) would share one XCD's CUs, so
   // all items then form one range.
   const int nranges = items.size() >= kRangeMinItems ? kItemRanges : 1;
-  std::vector<uint32_t> range(size_t(nranges) + 1, uint32_t(items.size()));
+  std::vector<uint32_t> range(size_t(nranges) + 1, npacks);
   range[0] = 0;
   if (nranges > 1) {
     int64_t acc = 0;
     int x = 1;
-    for (size_t k = 0; k < items.size() && x < nranges; ++k) {
-      acc += int64_t(items[k].end) - items[k].begin;
-      while (x < nranges && acc * nranges >= tot * x) range[size_t(x++)] = uint32_t(k + 1);
+    for (uint32_t k = 0; k < npacks && x < nranges; ++k) {
+      for (uint32_t i = packs[k]; i < packs[k + 1]; ++i) acc += int64_t(items[i].end) - items[i].begin;
+      while (x < nranges && acc * nranges >= tot * x) range[size_t(x++)] = k + 1;
     }
   }
   uint32_t* recs = P->alloc<uint32_t>(size_t(tot));
   BinItem* d_items = P->alloc<BinItem>(items.size());
   uint32_t* d_range = P->alloc<uint32_t>(range.size());
-  if (!recs || !d_items || !d_range) return fail(DDF_ENOMEM, "plan allocation failed");
+  uint32_t* d_packs = P->alloc<uint32_t>(packs.size());
+  if (!recs || !d_items || !d_range || !d_packs) return fail(DDF_ENOMEM, "plan allocation failed");
   if (!items.empty())
     HIP_TRY(hipMemcpyAsync(d_items, items.data(), items.size() * sizeof(BinItem), hipMemcpyHostToDevice, st));
   HIP_TRY(hipMemcpyAsync(d_range, range.data(), range.size() * 4, hipMemcpyHostToDevice, st));
-  *ranges_out = d_range;
-  *nranges_out = nranges;
+  HIP_TRY(hipMemcpyAsync(d_packs, packs.data(), packs.size() * 4, hipMemcpyHostToDevice, st));
+  p.pack_range = d_range;
+  p.pack_first = d_packs;
+  p.npacks = npacks;
+  p.nranges = nranges;
+  // degrid pass A: a workgroup of one wavefront where an item has few records for four
+  p.tile_threads = tot < int64_t(items.size()) * 192 ? 64 : 256;
   if (tile_first_out) {
     uint32_t* tf = P->alloc<uint32_t>(size_t(ntile_all));
     uint32_t* tc = P->alloc<uint32_t>(size_t(ntile_all));
@@ -1637,7 +1675,7 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   ddf_plan_opts o{};
   if (opts) o = *opts;
   const int tile = o.tile > 0 ? o.tile : 16;
-  const int chunk = o.chunk > 0 ? o.chunk : 2048;
+  const int chunk = o.chunk;
   const int halo = (maxsup - 1) / 2;
   {
     // the tile passes hold one (T + 2 h)^2 complex64 image per polarisation in LDS
@@ -1709,7 +1747,7 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     d.sum_jones_chan = f.jones.sum_jones_chan;
   }
   P->d_facets = P->alloc<FacetDev>(hf.size());
-  P->queues = P->alloc<uint32_t>(32);
+  P->queues = P->alloc<uint32_t>(ddf_plan::kQueues * kQueueStride);
   if (!P->d_facets || !P->queues) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
   if (hipMemcpyAsync(P->d_facets, hf.data(), hf.size() * sizeof(FacetDev), hipMemcpyHostToDevice, st) != hipSuccess)
     return bail(fail(DDF_EHIP, "plan upload failed"));
@@ -1773,8 +1811,7 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   // bins
   uint32_t ni = 0;
   int64_t nr = 0;
-  rc = build_bins(P, P->pg, P->vg, P->place_g, chunk, &P->recs_g, &P->items_g, &ni, &nr, &P->pg.item_range,
-                  &P->pg.nranges, true, st, &P->tile_first_g, &P->tile_count_g);
+  rc = build_bins(P, P->pg, P->vg, P->place_g, chunk, &P->recs_g, &P->items_g, &ni, &nr, true, st, &P->tile_first_g, &P->tile_count_g);
   if (rc) return bail(rc);
   P->pg.nitems_b = ni;
   P->stats[0] = nr;
@@ -1801,10 +1838,12 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     if (ni) {
       P->slots_g = P->alloc<float>(n);
       if (!P->slots_g) (void)hipGetLastError();
+      P->live_g = P->alloc<uint32_t>(1 + size_t(nfacets) * g->nband * P->pg.ntiles_y * P->pg.ntiles_x);
+      if (!P->live_g || batched_live_tiles(P->pg, P->tile_count_g, P->live_g, st))
+        return bail(fail(DDF_ENOMEM, "plan allocation failed"));
     }
   }
-  rc = build_bins(P, P->pd, P->vd, P->place_d, chunk, &P->recs_d, &P->items_d, &ni, &nr, &P->pd.item_range,
-                  &P->pd.nranges, false, st);
+  rc = build_bins(P, P->pd, P->vd, P->place_d, chunk, &P->recs_d, &P->items_d, &ni, &nr, false, st);
   if (rc) return bail(rc);
   P->pd.nitems_b = ni;
   P->stats[1] = nr;
@@ -1922,13 +1961,13 @@ extern "C" int ddf_plan_grid(ddf_plan* P, float* vis, int32_t dopsf, void* strea
   BatchParams p = P->pg;
   p.dopsf = dopsf;
   if (prepare_jones(P, st)) return fail(DDF_EHIP, "Jones preparation failed");
-  if (batched_reset(P->queues, 1 + kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
+  if (batched_reset(P->queue(0), 1 + kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
   P->mark(DDF_PASS_GRID_A, 0, st);
-  if (p.nitems_a && batched_grid_a(p, v, P->pcode_g, P->V, P->queues, P->nwg, st)) return fail(DDF_EHIP, "grid pass A launch failed");
+  if (p.nitems_a && batched_grid_a(p, v, P->pcode_g, P->V, P->queue(0), P->nwg, st)) return fail(DDF_EHIP, "grid pass A launch failed");
   P->mark(DDF_PASS_GRID_A, 1, st);
   P->mark(DDF_PASS_GRID_B, 0, st);
-  if (p.nitems_b && batched_grid_b(p, P->bstamp_g, P->V, P->items_g, P->recs_g, P->queues + 1, P->nwg_tiles[0], P->slots_g,
-                                     P->tile_first_g, P->tile_count_g, st))
+  if (p.nitems_b && batched_grid_b(p, P->bstamp_g, P->V, P->items_g, P->recs_g, P->queue(1), P->nwg_tiles[0], P->slots_g,
+                                     P->tile_first_g, P->tile_count_g, P->live_g, st))
     return fail(DDF_EHIP, "grid pass B launch failed");
   P->mark(DDF_PASS_GRID_B, 1, st);
   return DDF_OK;
@@ -1940,9 +1979,9 @@ extern "C" int ddf_plan_degrid(ddf_plan* P, float* vis, void* stream) {
   VisP v = P->vd;
   if (vis) v.vis = reinterpret_cast<float2*>(vis);
   if (prepare_jones(P, st)) return fail(DDF_EHIP, "Jones preparation failed");
-  if (batched_reset(P->queues + 1 + kItemRanges, kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
+  if (batched_reset(P->queue(1 + kItemRanges), kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
   P->mark(DDF_PASS_DEGRID_A, 0, st);
-  if (P->pd.nitems_b && batched_degrid_a(P->pd, P->bstamp_d, P->M, P->items_d, P->recs_d, P->queues + 1 + kItemRanges, P->nwg_tiles[1], st))
+  if (P->pd.nitems_b && batched_degrid_a(P->pd, P->bstamp_d, P->M, P->items_d, P->recs_d, P->queue(1 + kItemRanges), P->nwg_tiles[1], st))
     return fail(DDF_EHIP, "degrid pass A launch failed");
   P->mark(DDF_PASS_DEGRID_A, 1, st);
   P->mark(DDF_PASS_DEGRID_B, 0, st);
@@ -1956,14 +1995,14 @@ extern "C" int ddf_plan_degrid_adjoint(ddf_plan* P, const float* vis_bar, void* 
   if (!P || !vis_bar) return fail(DDF_EINVAL, "null argument");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (prepare_jones(P, st)) return fail(DDF_EHIP, "Jones preparation failed");
-  if (batched_reset(P->queues + 1 + 2 * kItemRanges, 1 + kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
+  if (batched_reset(P->queue(1 + 2 * kItemRanges), 1 + kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
   const float2* vb = reinterpret_cast<const float2*>(vis_bar);
   P->mark(DDF_PASS_ADJ_B, 0, st);
-  if (P->pd.nitems_a && batched_degrid_b_adjoint(P->pd, P->vd, P->pcode_d, vb, P->M, P->queues + 1 + 2 * kItemRanges, P->nwg, st))
+  if (P->pd.nitems_a && batched_degrid_b_adjoint(P->pd, P->vd, P->pcode_d, vb, P->M, P->queue(1 + 2 * kItemRanges), P->nwg, st))
     return fail(DDF_EHIP, "degrid adjoint pass B launch failed");
   P->mark(DDF_PASS_ADJ_B, 1, st);
   P->mark(DDF_PASS_ADJ_A, 0, st);
-  if (P->pd.nitems_b && batched_degrid_a_adjoint(P->pd, P->bstamp_d, P->M, P->items_d, P->recs_d, P->queues + 2 + 2 * kItemRanges, P->nwg_tiles[2], st))
+  if (P->pd.nitems_b && batched_degrid_a_adjoint(P->pd, P->bstamp_d, P->M, P->items_d, P->recs_d, P->queue(2 + 2 * kItemRanges), P->nwg_tiles[2], st))
     return fail(DDF_EHIP, "degrid adjoint pass A launch failed");
   P->mark(DDF_PASS_ADJ_A, 1, st);
   return DDF_OK;

@@ -230,7 +230,7 @@ typedef struct ddf_plan ddf_plan;
 
 typedef struct ddf_plan_opts {
   int32_t tile;            /* uv tile edge in grid cells (0: 16)                                */
-  int32_t chunk;           /* max records per tile work item (0: 2048)                          */
+  int32_t chunk;           /* max records per tile work item (0: 2048, fewer for small plans)    */
   int32_t blocks_per_item; /* BDA blocks per gridding work item (0: 128)                        */
   int32_t group;           /* facets per lane group in gridding (0: auto, <= 64)                */
   int32_t precision;       /* 0 mixed: FP64 uvw rotation and per-row phase base, FP32 sin/cos and
