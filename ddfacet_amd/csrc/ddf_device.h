@@ -330,6 +330,17 @@ __device__ inline JonesPair jones_at(const JonesP& jp, int64_t row, int chan, co
   return r;
 }
 
+// BB of a Jones pair: ((|J0_00| |J1_00| + |J0_11| |J1_11|) / 2)^2.
+__device__ __forceinline__ double jones_bb(cd x0, cd x1, cd y0, cd y1) {
+  // |x| |y| as sqrt(|x|^2 |y|^2): two square roots in place of four hypot calls, within an ulp or
+  // two of the product of the moduli.  The product of the squared moduli leaves the normal FP64
+  // range only where |x| |y| is above 1e154 or below 1e-154, where BB = bb^2 itself (nearly)
+  // overflows or underflows.
+  auto n2 = [](cd z) { return z.re * z.re + z.im * z.im; };
+  const double bb = (sqrt(n2(x0) * n2(y0)) + sqrt(n2(x1) * n2(y1))) / 2.;
+  return bb * bb;
+}
+
 // jones_at<true> for a key read beforehand: antennas a0 / a1, DD Jones time and channel kt / kc,
 // beam Jones time and channel bt / bc (the tables that are absent are not read).  No ScaleJones.
 __device__ __forceinline__ JonesPair jones_keyed(const JonesP& jp, int a0, int a1, int kt, int kc, int bt, int bc) {
@@ -345,14 +356,30 @@ __device__ __forceinline__ JonesPair jones_keyed(const JonesP& jp, int a0, int a
     r.J0 = prepared_jones(jp.pb, jp.bdims, bt, a0, jp.bdir, bc);
     r.J1 = prepared_jones(jp.pb, jp.bdims, bt, a1, jp.bdir, bc);
   }
-  // |x| |y| as sqrt(|x|^2 |y|^2): two square roots in place of four hypot calls, within an ulp or
-  // two of the product of the moduli.  The product of the squared moduli leaves the normal FP64
-  // range only where |x| |y| is above 1e154 or below 1e-154, where BB = bb^2 itself (nearly)
-  // overflows or underflows.
-  auto n2 = [](cd z) { return z.re * z.re + z.im * z.im; };
-  const double bb = (sqrt(n2(r.J0.a[0]) * n2(r.J1.a[0])) + sqrt(n2(r.J0.a[3]) * n2(r.J1.a[3]))) / 2.;
-  r.BB = bb * bb;
+  r.BB = jones_bb(r.J0.a[0], r.J0.a[3], r.J1.a[0], r.J1.a[3]);
   return r;
+}
+
+// Entry of direction 0 of a prepared table for (time, antenna, channel), in entries; the indices
+// clamped like give_jones.  prepared_at reads the entry of a direction.
+__device__ __forceinline__ uint32_t prepared_offset(const int* dims, int it, int ant, int ich) {
+  it = clampi(it, 0, dims[0] - 1);
+  ant = clampi(ant, 0, dims[2] - 1);
+  ich = clampi(ich, 0, dims[3] - 1);
+  return ((uint32_t(it) * uint32_t(dims[2]) + uint32_t(ant)) * uint32_t(dims[3]) + uint32_t(ich)) * uint32_t(dims[1]);
+}
+__device__ __forceinline__ M2 prepared_at(const double2* tab, const int* dims, uint32_t off, int dir) {
+  const DDF_GLOBAL double2* p = gptr(tab) + (size_t(off) + size_t(clampi(dir, 0, dims[1] - 1))) * 4;
+  M2 out;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) out.a[q] = cd{p[q].x, p[q].y};
+  return out;
+}
+// The Jones matrix of one antenna (DD times beam where both are given) from its table offsets.
+__device__ __forceinline__ M2 jones_from_offsets(const JonesP& jp, uint32_t k, uint32_t b, int kdir, int bdir) {
+  if (!jp.pk) return prepared_at(jp.pb, jp.bdims, b, bdir);
+  const M2 J = prepared_at(jp.pk, jp.kdims, k, kdir);
+  return jp.pb ? mul(J, prepared_at(jp.pb, jp.bdims, b, bdir)) : J;
 }
 
 // Entry of a prepared complex64 table (JonesP::pkf / pbf).

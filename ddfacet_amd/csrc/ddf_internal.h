@@ -232,6 +232,20 @@ struct BatchParams {
 constexpr int grid_a_key_offset(int read) { return (4 + 2 * read + 3) & ~3; }
 constexpr int grid_a_stride(int read) { return (grid_a_key_offset(read) + 12 + 3) & ~3; }
 
+// Visibilities of a map in the order in which grid pass A walks them (block by block, a block's channel
+// range cut where the Jones channel changes), for grid_pass_a_runs: entry = row | chan << 32 |
+// channels of its segment << 48 | opens a run of one Jones key << 63; start[b]: first entry of block b.
+struct RunList {
+  const uint64_t* entry;  // null: the map is gridded by grid_pass_a
+  const int64_t* start;   // [nblocks + 1]
+  int group, ngroups;     // facets of a group (per-channel sums in LDS), groups
+  const uint32_t* item;   // [nitems + 1] first block of a work item
+  uint32_t nitems;        // work items of a group: the blocks that start within `entries` entries
+  int64_t entries;
+  int chan_lds;
+  int jones32;  // one Jones table, whose complex64 copy is exact (neither interpolation nor NormJones changed it)
+};
+
 // host launchers (ddf_batched.hip)
 int batched_place(const BatchParams& p, const VisP& v, bool degrid, uint64_t* place, hipStream_t st);
 int batched_pair_codes(const uint64_t* place, int64_t n, uint8_t* code, hipStream_t st);
@@ -251,6 +265,16 @@ int batched_reset(uint32_t* counters, int n, hipStream_t st);
 size_t batched_grid_a_stage_bytes(int group, int read);
 int batched_grid_a(const BatchParams& p, const VisP& v, const uint8_t* pcode, float2* V, uint32_t* queue,
                    unsigned nwg, hipStream_t st);
+// Grid pass A on the run list (mixed precision, per-visibility Jones).  batched_runs_layout says whether
+// a plan takes it and sets the groups, batched_run_items the items of a list of `total` entries; queue: a
+// counter per group.
+constexpr int kRunQueues = 64;
+bool batched_runs_layout(const BatchParams& p, const VisP& v, int group, RunList* rl);
+void batched_run_split(int64_t total, RunList* rl);
+int batched_run_items(const VisP& v, const RunList& rl, uint32_t* item, hipStream_t st);
+int batched_grid_runs(const BatchParams& p, const VisP& v, const RunList& rl, const uint8_t* pcode, float2* V,
+                      uint32_t* queue, unsigned nwg, hipStream_t st);
+int batched_run_entries(const BatchParams& p, const VisP& v, const int64_t* start, uint64_t* entry, hipStream_t st);
 // slots: null -> tiles added into the grids with global atomics; else one tile slot per work item
 // ([nitems][npg][2][W*W]) and grid_slot_reduce (tile_first / tile_count: the items of each tile)
 int batched_grid_b(const BatchParams& p, const uint64_t* place, const float2* V, const BinItem* items,

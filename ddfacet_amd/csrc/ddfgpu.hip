@@ -1293,9 +1293,12 @@ struct ddf_plan {
   uint32_t* vrun = nullptr;       // run of each degrid list entry (block and Jones key shared)
   uint32_t* run_first = nullptr;  // first list entry of each run
   int64_t nruns = 0;
+  RunList runs = {};              // grid pass A on runs (entry null: grid_pass_a)
+  unsigned nwg_runs = 0;
   // work-queue counters (kQueueStride words apart): [0] grid pass A, [1, 9) grid pass B (one per item range), [9, 17) degrid
   // pass A, [17] the adjoint of degrid pass B, [18, 26) the adjoint of degrid pass A
-  static constexpr int kQueues = 2 + 3 * kItemRanges;
+  // [kQueueRuns ...) grid pass A on runs, one per facet group
+  static constexpr int kQueueRuns = 2 + 3 * kItemRanges, kQueues = kQueueRuns + kRunQueues;
   uint32_t* queues = nullptr;
   uint32_t* queue(int k) const { return queues + k * kQueueStride; }
   const float2* jsrc[2] = {nullptr, nullptr};  // caller's DD / beam Jones tables
@@ -1879,6 +1882,36 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
                    (size_t(nfacets) * per_f + size_t(G) * (2 * size_t(vgrid->nchan) + 1)) * 8 + stage_bytes <= 80 * 1024;
   if (size_t(nfacets) * per_f * 8 + stage_bytes > 80 * 1024)
     return bail(fail(DDF_EINVAL, "facets x bands too large for one plan"));
+  // the run list of the grid map
+  if (batched_runs_layout(P->pg, P->vg, o.group, &P->runs)) {
+    const int64_t nb = vgrid->nblocks;
+    Temp rt(st);
+    int32_t* cnt = static_cast<int32_t*>(rt.get(size_t(nb) * 4));
+    int64_t* tmp = static_cast<int64_t*>(rt.get(size_t((nb + kScanChunk - 1) / kScanChunk) * 8));
+    int64_t* start = P->alloc<int64_t>(size_t(nb) + 1);
+    if (!cnt || !tmp || !start) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+    if (batched_vis_counts(P->vg, cnt, st)) return bail(fail(DDF_EHIP, "launch failed"));
+    rc = launch_scan(cnt, nb, 0, start, tmp, st);
+    if (rc) return bail(rc);
+    int64_t last_start = 0;
+    int32_t last_cnt = 0;
+    if (hipMemcpyAsync(&last_start, start + nb - 1, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipMemcpyAsync(&last_cnt, cnt + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+      return bail(fail(DDF_EHIP, "copy failed"));
+    const int64_t total = last_start + last_cnt;
+    if (total >= (int64_t(1) << 36)) return bail(fail(DDF_EINVAL, "visibility list too long for one plan"));
+    uint64_t* entry = P->alloc<uint64_t>(size_t(total));
+    if (!entry || hipMemcpyAsync(start + nb, &total, 8, hipMemcpyHostToDevice, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess || batched_run_entries(P->pg, P->vg, start, entry, st))
+      return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+    P->runs.start = start;
+    batched_run_split(total, &P->runs);
+    uint32_t* item = P->alloc<uint32_t>(size_t(P->runs.nitems) + 1);
+    if (!item || batched_run_items(P->vg, P->runs, item, st)) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+    P->runs.item = item;
+    P->runs.entry = entry;
+  }
   // LDS tiles
   const int W = tile + 2 * halo;
   const int npg = smg.nstokes < g->npol ? smg.nstokes : g->npol;
@@ -1943,6 +1976,7 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
     return bail(fail(DDF_EHIP, "device query failed"));
   P->nwg = unsigned(o.workgroups > 0 ? o.workgroups : prop.multiProcessorCount * 4);
+  P->nwg_runs = unsigned(o.workgroups > 0 ? o.workgroups : prop.multiProcessorCount);
   if (o.workgroups > 0) {
     for (unsigned& x : P->nwg_tiles) x = unsigned(o.workgroups);
   } else if (batched_tile_wgs(P->pg, P->pd, P->nwg_tiles)) {
@@ -1962,7 +1996,12 @@ extern "C" int ddf_plan_grid(ddf_plan* P, float* vis, int32_t dopsf, void* strea
   p.dopsf = dopsf;
   if (prepare_jones(P, st)) return fail(DDF_EHIP, "Jones preparation failed");
   if (batched_reset(P->queue(0), 1 + kItemRanges, st)) return fail(DDF_EHIP, "launch failed");
+  if (P->runs.entry && batched_reset(P->queue(ddf_plan::kQueueRuns), P->runs.ngroups, st)) return fail(DDF_EHIP, "launch failed");
   P->mark(DDF_PASS_GRID_A, 0, st);
+  if (P->runs.entry) {
+    if (batched_grid_runs(p, v, P->runs, P->pcode_g, P->V, P->queue(ddf_plan::kQueueRuns), P->nwg_runs, st))
+      return fail(DDF_EHIP, "grid pass A launch failed");
+  } else
   if (p.nitems_a && batched_grid_a(p, v, P->pcode_g, P->V, P->queue(0), P->nwg, st)) return fail(DDF_EHIP, "grid pass A launch failed");
   P->mark(DDF_PASS_GRID_A, 1, st);
   P->mark(DDF_PASS_GRID_B, 0, st);
