@@ -110,16 +110,26 @@ __device__ __forceinline__ M2T<T> cvt(const M2T<U>& x) {
   return M2T<T>{{cvt<T>(x.a[0]), cvt<T>(x.a[1]), cvt<T>(x.a[2]), cvt<T>(x.a[3])}};
 }
 
-// ---- wavefront reductions (all lanes receive the total) ------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+// ---- wavefront reduction -------------------------------------------------------------------
+// The sum over the wavefront by row shifts and row broadcasts (DPP), a scalar: a step takes two moves and
+// an addition, against two LDS permutes of ~100 cycles in the butterfly.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(b)), CTRL, ROWS, 0xF, true));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), CTRL, ROWS, 0xF, true));
+  return v + __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
-__device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+__device__ __forceinline__ double wave_total(double v) {
+  v = dpp_add<0x111, 0xF>(v);  // row_shr 1, 2, 4, 8: lane 15 of a row has the row's sum
+  v = dpp_add<0x112, 0xF>(v);
+  v = dpp_add<0x114, 0xF>(v);
+  v = dpp_add<0x118, 0xF>(v);
+  v = dpp_add<0x142, 0xA>(v);  // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xC>(v);  // row_bcast 31 into rows 2 and 3: lane 63 has the sum
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b >> 32)), 63))) << 32) |
+                                        uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b)), 63)));
 }
 
 // ---- phasor ---------------------------------------------------------------------------------
