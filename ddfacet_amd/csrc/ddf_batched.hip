@@ -339,19 +339,31 @@ __global__ __launch_bounds__(256) void plan_stamp_records(BatchParams p, const u
 // Sp = S + (S & 1) (the pad cell is zero), plane pl at twice its put-order offset (a padded plane,
 // O2 S Sp cells, fits below twice the next plane's offset), so that every row starts on a 16-byte
 // boundary and a lane reads two cells per load.
-__global__ __launch_bounds__(256) void plan_cf_pad(const float2* in, float2* out, const int64_t* off,
-                                                   const int32_t* support, int nw, int overs) {
+__global__ __launch_bounds__(256) void plan_cf_pad(const FacetDev* facets, int nf, const int32_t* support, int nw, int overs) {
   const int pl = blockIdx.y;
   const int S = support[pl < nw ? pl : pl - nw];
   const int Sp = S + (S & 1);
   const int S2 = S * S, SSp = S * Sp, O2 = overs * overs;
-  const int64_t o = off[pl];
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < int64_t(O2) * SSp;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const int k = int(i / SSp);
-    const int rem = int(i - int64_t(k) * SSp);
-    const int r = rem / Sp, c = rem - r * Sp;
-    out[2 * o + i] = c < S ? in[o + int64_t(k) * S2 + r * S + c] : make_float2(0.f, 0.f);
+  for (int f = blockIdx.z; f < nf; f += gridDim.z) {
+    const FacetDev fd = gload(facets + f);
+    const DDF_GLOBAL float2* in = gptr(fd.cf);
+    DDF_GLOBAL float2* out = gptr_w(const_cast<float2*>(fd.cft));
+    const int64_t o = gptr(fd.cf_offset)[pl];
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < int64_t(O2) * SSp;
+         i += int64_t(gridDim.x) * blockDim.x) {
+      const int k = int(i / SSp);
+      const int rem = int(i - int64_t(k) * SSp);
+      const int r = rem / Sp, c = rem - r * Sp;
+      st2(out + (2 * o + i), c < S ? ld2(in + (o + int64_t(k) * S2 + r * S + c)) : make_float2(0.f, 0.f));
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void plan_cf_info(const CfSource* src, int nf, int nw, int32_t* support, int64_t* offset) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nf * 2 * nw; i += gridDim.x * blockDim.x) {
+    const int f = i / (2 * nw), k = i - f * 2 * nw;
+    offset[i] = src[f].offset[k];
+    if (k < nw) support[f * nw + k] = src[f].support[k];
   }
 }
 
@@ -2425,24 +2437,24 @@ int batched_sort_items(const BatchParams& p, const uint64_t* place, uint32_t* re
                        uint32_t nitems, bool stamp_order, hipStream_t st) {
   if (n <= 0 || nitems == 0) return DDF_OK;
   if (n >= (int64_t(1) << 31)) return DDF_EINVAL;
-  uint64_t *k0 = nullptr, *k1 = nullptr;
-  uint32_t *b0 = nullptr, *b1 = nullptr;
-  void* tmp = nullptr;
+  PoolArena arena;
   size_t tb = 0;
   int rc = DDF_OK;
   auto grid = [](int64_t m) { int64_t g = (m + 255) / 256; return unsigned(g > 65536 ? 65536 : (g < 1 ? 1 : g)); };
-  if (hipMallocAsync(reinterpret_cast<void**>(&k0), size_t(n) * 8, st) != hipSuccess ||
-      hipMallocAsync(reinterpret_cast<void**>(&k1), size_t(n) * 8, st) != hipSuccess ||
-      hipMallocAsync(reinterpret_cast<void**>(&b0), size_t(nitems) * 4, st) != hipSuccess ||
-      hipMallocAsync(reinterpret_cast<void**>(&b1), size_t(nitems) * 4, st) != hipSuccess) {
+  uint64_t* k0 = static_cast<uint64_t*>(arena.get(size_t(n) * 8, st));
+  uint64_t* k1 = static_cast<uint64_t*>(arena.get(size_t(n) * 8, st));
+  uint32_t* b0 = static_cast<uint32_t*>(arena.get(size_t(nitems) * 4, st));
+  uint32_t* b1 = static_cast<uint32_t*>(arena.get(size_t(nitems) * 4, st));
+  if (!k0 || !k1 || !b0 || !b1) {
     rc = DDF_ENOMEM;
   } else {
     if (stamp_order) hipLaunchKernelGGL(plan_sort_keys<true>, dim3(grid(n)), dim3(256), 0, st, p, place, recs, n, k0);
     else hipLaunchKernelGGL(plan_sort_keys<false>, dim3(grid(n)), dim3(256), 0, st, p, place, recs, n, k0);
     hipLaunchKernelGGL(plan_item_bounds, dim3(grid(nitems)), dim3(256), 0, st, items, nitems, b0, b1);
+    void* tmp = nullptr;
     if (hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, tb, k0, k1, int(n), int(nitems), b0, b1, 0, 51, st) !=
             hipSuccess ||
-        hipMallocAsync(&tmp, tb ? tb : 1, st) != hipSuccess ||
+        !(tmp = arena.get(tb, st)) ||
         hipcub::DeviceSegmentedRadixSort::SortKeys(tmp, tb, k0, k1, int(n), int(nitems), b0, b1, 0, 51, st) !=
             hipSuccess) {
       rc = DDF_EHIP;
@@ -2451,11 +2463,7 @@ int batched_sort_items(const BatchParams& p, const uint64_t* place, uint32_t* re
       if (hipGetLastError() != hipSuccess) rc = DDF_EHIP;
     }
   }
-  if (tmp) hipFreeAsync(tmp, st);
-  if (k0) hipFreeAsync(k0, st);
-  if (k1) hipFreeAsync(k1, st);
-  if (b0) hipFreeAsync(b0, st);
-  if (b1) hipFreeAsync(b1, st);
+  arena.release_all(st);
   return rc;
 }
 
@@ -2774,14 +2782,20 @@ int batched_degrid_b_adjoint(const BatchParams& p, const VisP& v, const uint8_t*
 
 namespace ddf {
 
-int batched_cf_pad(const float2* in, float2* out, const int64_t* off, const int32_t* support, int nw, int overs,
-                   int max_support, hipStream_t st) {
+int batched_cf_pad(const FacetDev* facets, int nf, const int32_t* support, int nw, int overs, int max_support,
+                   hipStream_t st) {
   const int64_t n = int64_t(overs) * overs * max_support * (max_support + 1);
   int64_t nb = (n + 255) / 256;
   if (nb > 1024) nb = 1024;
   if (nb < 1) nb = 1;
-  hipLaunchKernelGGL(plan_cf_pad, dim3(unsigned(nb), unsigned(2 * nw)), dim3(256), 0, st, in, out, off, support, nw,
-                     overs);
+  hipLaunchKernelGGL(plan_cf_pad, dim3(unsigned(nb), unsigned(2 * nw), unsigned(std::min(nf, 65535))), dim3(256), 0, st, facets,
+                     nf, support, nw, overs);
+  return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
+}
+
+int batched_cf_info(const CfSource* src, int nf, int nw, int32_t* support, int64_t* offset, hipStream_t st) {
+  hipLaunchKernelGGL(plan_cf_info, dim3(unsigned(std::min(1024, (nf * 2 * nw + 255) / 256))), dim3(256), 0, st, src, nf, nw,
+                     support, offset);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
 }
 

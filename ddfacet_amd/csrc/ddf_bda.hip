@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "../../include/ddfgpu.h"
+#include "ddf_pool.h"
 
 namespace ddf {
 void set_last_error(const std::string& msg);  // ddfgpu.hip: the message ddf_last_error() returns
@@ -326,20 +327,18 @@ struct ddf_bda_builder {
   int64_t nrow = 0, nblk = 0, nwords = 0;
   const double* uvw = nullptr;
   const int32_t* chan_map = nullptr;
-  std::vector<void*> allocs;
+  ddf::PoolArena arena;
   uint32_t* rows = nullptr;   // sorted rows
   int64_t* seg = nullptr;
   int64_t* blk_off = nullptr;
   int64_t* word_off = nullptr;
   ~ddf_bda_builder() {
-    for (void* p : allocs) (void)hipFree(p);
+    if (!arena.empty()) (void)hipDeviceSynchronize();
+    arena.release_all(nullptr);
   }
   template <typename T>
   T* alloc(size_t n) {
-    void* p = nullptr;
-    if (hipMalloc(&p, (n ? n : 1) * sizeof(T)) != hipSuccess) return nullptr;
-    allocs.push_back(p);
-    return static_cast<T*>(p);
+    return static_cast<T*>(arena.get(std::max<size_t>(n, 1) * sizeof(T), st));
   }
 };
 
@@ -453,7 +452,7 @@ extern "C" int ddf_bda_build_write(ddf_bda_builder* B, int32_t* out, int64_t n, 
   if (n < B->nwords) return bfail(DDF_EINVAL, "output shorter than the map");
   hipStream_t st = static_cast<hipStream_t>(stream);
   BlockDesc* desc = nullptr;
-  hipError_t ea = hipMallocAsync(reinterpret_cast<void**>(&desc), size_t(B->nblk ? B->nblk : 1) * sizeof(BlockDesc), st);
+  hipError_t ea = ddf::pool_alloc(reinterpret_cast<void**>(&desc), size_t(B->nblk ? B->nblk : 1) * sizeof(BlockDesc), st);
   if (ea != hipSuccess) return bfail(DDF_EHIP, std::string("BDA descriptors: ") + hipGetErrorString(ea));
   const BdaParams& P = B->P;
   if (P.mode == 1)

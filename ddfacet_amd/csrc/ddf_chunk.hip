@@ -16,6 +16,7 @@
 #include <string>
 
 #include "../../include/ddfgpu.h"
+#include "ddf_pool.h"
 
 namespace ddf {
 void set_last_error(const std::string& msg);  // ddfgpu.hip: the message ddf_last_error() returns
@@ -149,11 +150,11 @@ extern "C" int ddf_sort_baseline_time(const int32_t* a0, const int32_t* a1, cons
   void* tmp = nullptr;
   size_t tb1 = 0, tb2 = 0;
   const int n = int(nrow);
-  CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&tk), size_t(n) * 8, st));
-  CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&tk2), size_t(n) * 8, st));
-  CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&pk), size_t(n) * 4, st));
-  CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&pk2), size_t(n) * 4, st));
-  CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&perm2), size_t(n) * 4, st));
+  CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&tk), size_t(n) * 8, st));
+  CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&tk2), size_t(n) * 8, st));
+  CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&pk), size_t(n) * 4, st));
+  CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&pk2), size_t(n) * 4, st));
+  CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&perm2), size_t(n) * 4, st));
   hipLaunchKernelGGL(copy_f64_k, dim3(grid_for(n)), dim3(256), 0, st, times, tk, int64_t(n));
   hipLaunchKernelGGL(iota_k, dim3(grid_for(n)), dim3(256), 0, st, index, int64_t(n));
   {
@@ -164,7 +165,7 @@ extern "C" int ddf_sort_baseline_time(const int32_t* a0, const int32_t* a1, cons
     hipcub::DoubleBuffer<uint32_t> k2(pk, pk2);
     hipcub::DoubleBuffer<int32_t> v2(index, perm2);
     CHUNK_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb2, k2, v2, n, 0, 32, st));
-    CHUNK_TRY(hipMallocAsync(&tmp, tb1 > tb2 ? tb1 : tb2, st));
+    CHUNK_TRY(ddf::pool_alloc(&tmp, tb1 > tb2 ? tb1 : tb2, st));
     CHUNK_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, tb1, k1, v1, n, 0, 64, st));
     // pass 2: by antenna pair over the time order (stable: time, then row, among equal pairs)
     int32_t* p1 = v1.Current();
@@ -210,10 +211,10 @@ extern "C" int ddf_flag_selection(uint8_t* flags, const double* uvw, const doubl
   int rc = DDF_OK;
   unsigned long long* cnt = nullptr;
   uint8_t* named = nullptr;
-  CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&cnt), size_t(2 * na) * 8, st));
+  CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&cnt), size_t(2 * na) * 8, st));
   CHUNK_TRY(hipMemsetAsync(cnt, 0, size_t(2 * na) * 8, st));
   if (sel->named_antennas) {
-    CHUNK_TRY(hipMallocAsync(reinterpret_cast<void**>(&named), size_t(na), st));
+    CHUNK_TRY(ddf::pool_alloc(reinterpret_cast<void**>(&named), size_t(na), st));
     CHUNK_TRY(hipMemcpyAsync(named, sel->named_antennas, size_t(na), hipMemcpyHostToDevice, st));
   }
   if (nrow > 0)

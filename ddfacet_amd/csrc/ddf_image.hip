@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/ddfgpu.h"
+#include "ddf_pool.h"
 #include "ddf_device.h"
 #include "ddf_fft.h"
 
@@ -634,7 +635,7 @@ int upload_facets(const ddf_image_facet* facets, int nf, int n, int m, hipStream
       return ifail(DDF_EINVAL, "facet box does not intersect the main image consistently");
   }
   void* d = nullptr;
-  HIP_OK(hipMallocAsync(&d, h.size() * sizeof(ImgFacet), st));
+  HIP_OK(ddf::pool_alloc(&d, h.size() * sizeof(ImgFacet), st));
   tmp.push_back(d);
   HIP_OK(hipMemcpyAsync(d, h.data(), h.size() * sizeof(ImgFacet), hipMemcpyHostToDevice, st));
   *dout = static_cast<ImgFacet*>(d);
@@ -716,11 +717,11 @@ struct FFTCall {
   }
   // tmp of `total` values and what the plan wants
   int setup(FFTPlan* P, int64_t total) {
-    HIP_OK(hipMallocAsync(&tmp, size_t(total) * sizeof(float2), st));
+    HIP_OK(ddf::pool_alloc(&tmp, size_t(total) * sizeof(float2), st));
     if (rocfft_execution_info_create(&info) != rocfft_status_success)
       return ifail(DDF_EHIP, "rocfft_execution_info_create failed");
     if (P->work_size) {
-      HIP_OK(hipMallocAsync(&work, P->work_size, st));
+      HIP_OK(ddf::pool_alloc(&work, P->work_size, st));
       if (rocfft_execution_info_set_work_buffer(info, work, P->work_size) != rocfft_status_success)
         return ifail(DDF_EHIP, "rocfft work buffer failed");
     }
@@ -824,7 +825,7 @@ extern "C" int ddf_stitch(const ddf_image_facet* facets, int32_t nf, int32_t npi
   if (rc) return rc;
   // "if (FacetNorm != 0).any(): Image /= FacetNorm"
   int* flag = nullptr;
-  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&flag), sizeof(int), st));
+  HIP_OK(ddf::pool_alloc(reinterpret_cast<void**>(&flag), sizeof(int), st));
   tmp.push_back(flag);
   hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, st, flag, 1);
   hipLaunchKernelGGL(any_nonzero_kernel, dim3(unsigned(std::min<int64_t>(256, 1 + int64_t(m) * m / 16384))), dim3(256), 0, st, facet_norm,
@@ -848,7 +849,7 @@ extern "C" int ddf_model_to_grid(const ddf_image_facet* facets, int32_t nf, int3
   if (rc) return rc;
   const int n = npix_facet, per = nband * npol;
   int* nz = nullptr;
-  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&nz), sizeof(int) * size_t(per) * nf, st));
+  HIP_OK(ddf::pool_alloc(reinterpret_cast<void**>(&nz), sizeof(int) * size_t(per) * nf, st));
   tmp.push_back(nz);
   const float factor = float(double(overs) * n) * float(double(overs) * n);
   const CutP cut{image, facet_norm, nz, m, per, factor};

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "ddf_device.h"
+#include "ddf_pool.h"
 
 namespace ddf {
 
@@ -301,10 +302,16 @@ int batched_tile_wgs(const BatchParams& pg, const BatchParams& pd, unsigned out[
 // stamp records (tile offset | support << 16 | CF offset << 32) of the binned records
 int batched_stamp_records(const BatchParams& p, const uint64_t* place, const uint32_t* recs, int64_t n,
                           uint64_t* bstamp, hipStream_t st);
-// CF planes of one facet copied for degrid pass A: plane p (offset off[p], support S =
+// CF planes of every facet copied for degrid pass A (FacetDev::cft): plane p (offset off[p], support S =
 // support[p mod nw]) at offset 2 off[p], each sub-kernel's S rows padded to an even pitch with zeros
-int batched_cf_pad(const float2* in, float2* out, const int64_t* off, const int32_t* support, int nw, int overs,
-                   int max_support, hipStream_t st);
+int batched_cf_pad(const FacetDev* facets, int nf, const int32_t* support, int nw, int overs, int max_support,
+                   hipStream_t st);
+// the supports [nf][nw] and plane offsets [nf][2 nw] of every facet's CF table, side by side
+struct CfSource {
+  const int32_t* support;
+  const int64_t* offset;
+};
+int batched_cf_info(const CfSource* src, int nf, int nw, int32_t* support, int64_t* offset, hipStream_t st);
 int batched_prepare_jones(const BatchParams& p, const float2* src, double2* dst, float2* dstf, int dd, hipStream_t st);
 
 }  // namespace ddf

@@ -20,6 +20,7 @@
 #include <string>
 
 #include "../../include/ddfgpu.h"
+#include "ddf_pool.h"
 
 namespace ddf {
 void set_last_error(const std::string& msg);  // ddfgpu.hip: the message ddf_last_error() returns
@@ -207,7 +208,7 @@ int ddf_beam_jones(const ddf_beam_desc* b, const double* ra, const double* dec, 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t nmean = int64_t(ndir + 1) * b->nchan_jones;
   double* mean = nullptr;
-  if (hipMallocAsync(reinterpret_cast<void**>(&mean), size_t(nmean) * sizeof(double), st) != hipSuccess)
+  if (ddf::pool_alloc(reinterpret_cast<void**>(&mean), size_t(nmean) * sizeof(double), st) != hipSuccess)
     return jfail(DDF_ENOMEM, "ddf_beam_jones: workspace allocation failed");
   hipLaunchKernelGGL(beam_mean_k, dim3(blocks_for(nmean)), dim3(256), 0, st, *b, ra, dec, ndir, ra_c, dec_c, mean);
   const int64_t nout = int64_t(ntime) * ndir * na * b->nchan_jones;

@@ -793,17 +793,10 @@ void fill_params(KParams& p, const ddf_grid_desc* g, const ddf_vis* v, const ddf
 // Per-call temporary device memory (stream ordered).
 struct Temp {
   hipStream_t st;
-  std::vector<void*> ptrs;
+  PoolArena arena;
   explicit Temp(hipStream_t s) : st(s) {}
-  void* get(size_t bytes) {
-    void* p = nullptr;
-    if (hipMallocAsync(&p, bytes, st) != hipSuccess) return nullptr;
-    ptrs.push_back(p);
-    return p;
-  }
-  ~Temp() {
-    for (void* p : ptrs) (void)hipFreeAsync(p, st);
-  }
+  void* get(size_t bytes) { return arena.get(bytes, st); }
+  ~Temp() { arena.release_all(st); }
 };
 
 int resolve_block_index(const ddf_vis* v, Temp& tmp, const int64_t** out) {
@@ -901,6 +894,43 @@ int launch_degrid_r(const KParams& p, int jmode, int lg, unsigned nb, hipStream_
 
 namespace ddf {
 void set_last_error(const std::string& msg) { g_err = msg; }
+
+hipError_t pool_alloc(void** p, size_t bytes, hipStream_t st) {
+  static std::mutex mu;
+  static hipMemPool_t pools[64] = {};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= 64) return hipMallocAsync(p, bytes, st);
+  hipMemPool_t pool;
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    if (!pools[dev]) {
+      hipMemPoolProps props;
+      std::memset(&props, 0, sizeof(props));
+      props.allocType = hipMemAllocationTypePinned;
+      props.location.type = hipMemLocationTypeDevice;
+      props.location.id = dev;
+      hipMemPool_t made = nullptr;
+      e = hipMemPoolCreate(&made, &props);
+      if (e != hipSuccess) return e;
+      uint64_t keep = kPoolKeep;
+      e = hipMemPoolSetAttribute(made, hipMemPoolAttrReleaseThreshold, &keep);
+      if (e != hipSuccess) {
+        (void)hipMemPoolDestroy(made);
+        return e;
+      }
+      pools[dev] = made;
+    }
+    pool = pools[dev];
+  }
+  e = hipMallocFromPoolAsync(p, bytes, pool, st);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  (void)hipStreamSynchronize(st);
+  (void)hipMemPoolTrimTo(pool, 0);
+  return hipMallocFromPoolAsync(p, bytes, pool, st);
+}
 }  // namespace ddf
 
 // ---- Briggs transform without allocation ------------------------------------------------------
@@ -1422,13 +1452,16 @@ struct ddf_plan {
   unsigned nwg = 0;
   unsigned nwg_tiles[3] = {0, 0, 0};  // tile passes (grid B, degrid A, adjoint): as many as fit
   int64_t stats[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  std::vector<void*> allocs;
+  PoolArena arena;
+  hipStream_t st = nullptr;       // the stream of the build
   // per-pass timing (ddf_plan_timing): events around each pass on the launch stream
   int timing = 0;
   hipEvent_t ev[DDF_PLAN_NPASS][2] = {};
   int ev_set[DDF_PLAN_NPASS] = {};
   ~ddf_plan() {
-    for (void* p : allocs) (void)hipFree(p);
+    // a cycle may still be under way on any stream
+    if (!arena.empty()) (void)hipDeviceSynchronize();
+    arena.release_all(nullptr);
     for (auto& e : ev)
       for (hipEvent_t x : e)
         if (x) (void)hipEventDestroy(x);
@@ -1440,25 +1473,16 @@ struct ddf_plan {
   }
   template <typename T>
   T* alloc(size_t n) {
-    void* p = nullptr;
-    size_t bytes = n * sizeof(T);
-    if (bytes == 0) bytes = sizeof(T);
-    if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
-    allocs.push_back(p);
-    stats[5] += int64_t(bytes);
+    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+    void* p = arena.get(bytes, st);
+    if (p) stats[5] += int64_t(bytes);
     return static_cast<T*>(p);
   }
-  // frees one allocation of this plan (bytes as allocated)
+  // frees one allocation of this plan (bytes as allocated) once the stream of the build is through with it
   template <typename T>
   void release(T*& p, size_t n) {
-    for (size_t k = 0; k < allocs.size(); ++k) {
-      if (allocs[k] != static_cast<void*>(p)) continue;
-      (void)hipFree(allocs[k]);
-      allocs[k] = allocs.back();
-      allocs.pop_back();
-      stats[5] -= int64_t(n ? n * sizeof(T) : sizeof(T));
-      break;
-    }
+    arena.release(p, st);
+    stats[5] -= int64_t(std::max<size_t>(n, 1) * sizeof(T));
     p = nullptr;
   }
 };
@@ -1730,31 +1754,48 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
       (vdegrid->nblocks + 1) * int64_t(nfacets) >= (int64_t(1) << 32))
     return fail(DDF_EINVAL, "blocks x facets exceeds the 32-bit record index");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // shared CF geometry
-  std::vector<int32_t> sup0(static_cast<size_t>(c0.nw)), supi(static_cast<size_t>(c0.nw));
-  HIP_TRY(hipMemcpyAsync(sup0.data(), c0.support, sup0.size() * 4, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
+  // shared CF geometry: every facet's supports and plane offsets read back together
+  for (int i = 1; i < nfacets; ++i) {
+    const ddf_cf& ci = facets[i].cf;
+    if (ci.nw != c0.nw || ci.overs != c0.overs || ci.ref_wave != c0.ref_wave || ci.wmax != c0.wmax)
+      return fail(DDF_EINVAL, "all facets of a plan must share nw, OverS, RefWave and wmax");
+    if (!ci.data || !ci.offset || !ci.support) return fail(DDF_EINVAL, "bad CF table");
+    if (!facets[i].grid || !models[i] || !facets[i].sumwt) return fail(DDF_EINVAL, "facet buffer is null");
+    if (facets[0].jones.enabled && (!facets[i].jones.sum_jones || !facets[i].jones.sum_jones_chan))
+      return fail(DDF_EINVAL, "SumJones buffers are null");
+  }
+  const size_t nw0 = size_t(c0.nw);
+  std::vector<int32_t> sups(size_t(nfacets) * nw0);
+  std::vector<int64_t> offs(size_t(nfacets) * 2 * nw0);
+  {
+    Temp ct(st);
+    std::vector<CfSource> src(static_cast<size_t>(nfacets));
+    for (int i = 0; i < nfacets; ++i) src[size_t(i)] = CfSource{facets[i].cf.support, facets[i].cf.offset};
+    CfSource* d_src = static_cast<CfSource*>(ct.get(src.size() * sizeof(CfSource)));
+    int32_t* d_sup = static_cast<int32_t*>(ct.get(sups.size() * 4));
+    int64_t* d_off = static_cast<int64_t*>(ct.get(offs.size() * 8));
+    if (!d_src || !d_sup || !d_off) return fail(DDF_ENOMEM, "plan allocation failed");
+    HIP_TRY(hipMemcpyAsync(d_src, src.data(), src.size() * sizeof(CfSource), hipMemcpyHostToDevice, st));
+    if (batched_cf_info(d_src, nfacets, c0.nw, d_sup, d_off, st)) return fail(DDF_EHIP, "reading the CF tables failed");
+    HIP_TRY(hipMemcpyAsync(sups.data(), d_sup, sups.size() * 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(offs.data(), d_off, offs.size() * 8, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+  }
+  const std::vector<int32_t> sup0(sups.begin(), sups.begin() + c0.nw);
   int maxsup = 0;
   for (int32_t x : sup0) {
     if (x <= 0 || x % 2 == 0) return fail(DDF_EINVAL, "CF supports must be odd and positive");
     maxsup = x > maxsup ? x : maxsup;
   }
-  for (int i = 1; i < nfacets; ++i) {
-    const ddf_cf& ci = facets[i].cf;
-    if (ci.nw != c0.nw || ci.overs != c0.overs || ci.ref_wave != c0.ref_wave || ci.wmax != c0.wmax)
-      return fail(DDF_EINVAL, "all facets of a plan must share nw, OverS, RefWave and wmax");
-    HIP_TRY(hipMemcpyAsync(supi.data(), ci.support, supi.size() * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    if (supi != sup0) return fail(DDF_EINVAL, "all facets of a plan must share the CF supports");
-    if (!facets[i].grid || !models[i] || !facets[i].sumwt) return fail(DDF_EINVAL, "facet buffer is null");
-    if (facets[0].jones.enabled && (!facets[i].jones.sum_jones || !facets[i].jones.sum_jones_chan))
-      return fail(DDF_EINVAL, "SumJones buffers are null");
-  }
+  for (int i = 1; i < nfacets; ++i)
+    if (!std::equal(sup0.begin(), sup0.end(), sups.begin() + size_t(i) * nw0))
+      return fail(DDF_EINVAL, "all facets of a plan must share the CF supports");
   if (!models[0] || !facets[0].sumwt) return fail(DDF_EINVAL, "facet buffer is null");
   if (facets[0].jones.enabled && (!facets[0].jones.sum_jones || !facets[0].jones.sum_jones_chan))
     return fail(DDF_EINVAL, "SumJones buffers are null");
 
   ddf_plan* P = new ddf_plan();
+  P->st = st;
   auto bail = [&](int code) {
     delete P;
     return code;
@@ -1820,36 +1861,32 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   P->d_support = P->alloc<int32_t>(sup0.size());
   if (!P->d_support || hipMemcpyAsync(P->d_support, sup0.data(), sup0.size() * 4, hipMemcpyHostToDevice, st) != hipSuccess)
     return bail(fail(DDF_EHIP, "plan upload failed"));
+  // padded copies of the facets' CF planes for degrid pass A (rows of an even pitch, plane pl at twice its
+  // offset), all in one buffer, each at an even element
+  std::vector<size_t> pad(size_t(nfacets) + 1, 0);
+  for (int i = 0; i < nfacets; ++i) {
+    int64_t total = 0, total_pad = 0;
+    for (int pl = 0; pl < 2 * c0.nw; ++pl) {
+      const int64_t S = sup0[size_t(pl < c0.nw ? pl : pl - c0.nw)], O2 = int64_t(c0.overs) * c0.overs;
+      const int64_t off = offs[size_t(i) * 2 * nw0 + size_t(pl)];
+      total = std::max(total, off + O2 * S * S);
+      total_pad = std::max(total_pad, 2 * off + O2 * S * (S + (S & 1)));
+    }
+    // grid pass B addresses a facet's CF values by a 32-bit byte offset
+    if (total * int64_t(sizeof(float2)) >= (int64_t(1) << 32))
+      return bail(fail(DDF_EINVAL, "a facet's CF table reaches 4 GiB"));
+    pad[size_t(i) + 1] = pad[size_t(i)] + size_t(total_pad + (total_pad & 1));
+  }
+  float2* padded = P->alloc<float2>(pad.back());
+  if (!padded) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
   std::vector<FacetDev> hf(static_cast<size_t>(nfacets));
   for (int i = 0; i < nfacets; ++i) {
     const ddf_facet& f = facets[i];
     FacetDev& d = hf[size_t(i)];
+    d.cft = padded + pad[size_t(i)];
     d.grid = f.grid;
     d.model = models[i];
     d.cf = reinterpret_cast<const float2*>(f.cf.data);
-    {
-      // padded copy of the facet's CF planes for degrid pass A: rows of an even pitch, plane pl at
-      // twice its offset
-      const int nw = f.cf.nw, ov = f.cf.overs;
-      std::vector<int64_t> off(size_t(2 * nw));
-      if (hipMemcpyAsync(off.data(), f.cf.offset, off.size() * 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
-          hipStreamSynchronize(st) != hipSuccess)
-        return bail(fail(DDF_EHIP, "reading the CF plane offsets failed"));
-      int64_t total = 0, total_pad = 0;
-      for (int pl = 0; pl < 2 * nw; ++pl) {
-        const int64_t S = sup0[size_t(pl < nw ? pl : pl - nw)];
-        total = std::max(total, off[size_t(pl)] + int64_t(ov) * ov * S * S);
-        total_pad = std::max(total_pad, 2 * off[size_t(pl)] + int64_t(ov) * ov * S * (S + (S & 1)));
-      }
-      // grid pass B addresses a facet's CF values by a 32-bit byte offset
-      if (total * int64_t(sizeof(float2)) >= (int64_t(1) << 32))
-        return bail(fail(DDF_EINVAL, "a facet's CF table reaches 4 GiB"));
-      float2* t = P->alloc<float2>(size_t(total_pad));
-      if (!t) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-      if (batched_cf_pad(d.cf, t, f.cf.offset, P->d_support, nw, ov, maxsup, st))
-        return bail(fail(DDF_EHIP, "CF copy launch failed"));
-      d.cft = t;
-    }
     d.cf_offset = f.cf.offset;
     d.cu = f.cu;
     d.cv = f.cv;
@@ -1869,6 +1906,8 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   if (!P->d_facets || !P->queues) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
   if (hipMemcpyAsync(P->d_facets, hf.data(), hf.size() * sizeof(FacetDev), hipMemcpyHostToDevice, st) != hipSuccess)
     return bail(fail(DDF_EHIP, "plan upload failed"));
+  if (batched_cf_pad(P->d_facets, nfacets, P->d_support, c0.nw, c0.overs, maxsup, st))
+    return bail(fail(DDF_EHIP, "CF copy launch failed"));
   for (BatchParams* bp : {&P->pg, &P->pd}) {
     bp->facets = P->d_facets;
     bp->nf = nfacets;
