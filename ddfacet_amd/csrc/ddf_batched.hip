@@ -1994,6 +1994,63 @@ struct RunInfo {
   JonesKey key;        // the Jones key of the run (complex64 Jones tables only)
 };
 
+// The run that starts at list entry kr.
+template <int JMODE>
+__device__ __forceinline__ RunInfo degrid_run(const BatchParams& p, const VisP& v, const uint64_t* vrc,
+                                              const uint32_t* vblk, uint32_t kr, int64_t nvl, bool keyed) {
+  RunInfo ri;
+  ri.row = -1;
+  ri.chan = 0;
+  ri.mid = -1;
+  ri.blk = 0;
+  ri.tscale = 0;
+  ri.key = JonesKey{0, 0, 0, 0, 0, 0};
+  if (int64_t(kr) >= nvl) return ri;
+  const uint64_t e = vrc[kr];
+  const int64_t row = int64_t(uint32_t(e));
+  const int chan = int(e >> 32);
+  const uint32_t rb = vblk[kr];
+  if (!(row >= 0 && row < v.nrow && chan >= 0 && chan < v.nchan && int64_t(rb) < v.nblocks)) return ri;
+  ri.row = int(row);
+  ri.chan = chan;
+  ri.blk = rb;
+  if (JMODE == 2 || p.dp.enabled) {
+    const BlockRec br = read_block(v, rb);
+    double fm = 0;
+    for (int cc = br.ch0; cc < br.ch1; ++cc) fm += gptr(v.freqs)[cc];
+    if (br.ch1 > br.ch0) fm /= double(br.ch1 - br.ch0);
+    ri.tscale = decorr_tscale(fm);
+    if (br.nr > 0) {
+      const int64_t mid = br.rows[br.nr / 2];
+      if (mid >= 0 && mid < v.nrow) ri.mid = int(mid);
+    }
+    if (JMODE == 2) ri.chan = (br.ch0 + br.ch1) / 2;
+  }
+  const int jrow = JMODE == 2 ? ri.mid : ri.row;
+  if (keyed && jrow >= 0) ri.key = jones_key_f(p.jp, jrow, ri.chan);
+  return ri;
+}
+
+// residual of visibility (row, c): its value less acc
+template <int NCORR>
+__device__ __forceinline__ void degrid_residual(const VisP& v, int64_t row, int c, const cd (&acc)[4]) {
+  DDF_GLOBAL float2* vp = gptr_w(v.vis) + (size_t(row) * v.nchan + c) * NCORR;
+  if (NCORR == 4) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float2 x = ld2(vp + q);
+      st2(vp + q, make_float2(float(double(x.x) - acc[q].re), float(double(x.y) - acc[q].im)));
+    }
+  } else if (NCORR == 2) {
+    const float2 x0 = ld2(vp), x1 = ld2(vp + 1);
+    st2(vp, make_float2(float(double(x0.x) - acc[0].re), float(double(x0.y) - acc[0].im)));
+    st2(vp + 1, make_float2(float(double(x1.x) - acc[3].re), float(double(x1.y) - acc[3].im)));
+  } else {
+    const float2 x0 = ld2(vp);
+    st2(vp, make_float2(float(double(x0.x) - acc[0].re), float(double(x0.y) - acc[0].im)));
+  }
+}
+
 template <int NCORR, int JMODE, int PREC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void degrid_pass_b(BatchParams p, const VisP v, const float2* M,
                                                      const uint64_t* vrc, const uint32_t* vblk,
@@ -2025,40 +2082,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
     const int nr = int(vrun[klast] - r0) + 1;  // runs of the tile (at most 256)
     // run table of the tile
     if (t < nr) {
-      RunInfo ri;
-      ri.row = -1;
-      ri.chan = 0;
-      ri.mid = -1;
-      ri.blk = 0;
-      ri.tscale = 0;
-      ri.key = JonesKey{0, 0, 0, 0, 0, 0};
-      const uint32_t kr = run_first[r0 + t];
-      if (int64_t(kr) < nvl) {
-        const uint64_t e = vrc[kr];
-        const int64_t rrow = int64_t(uint32_t(e));
-        const int rc_ = int(e >> 32);
-        const uint32_t rb = vblk[kr];
-        if (rrow >= 0 && rrow < v.nrow && rc_ >= 0 && rc_ < v.nchan && int64_t(rb) < v.nblocks) {
-          ri.row = int(rrow);
-          ri.chan = rc_;
-          ri.blk = rb;
-          if (JMODE == 2 || p.dp.enabled) {
-            const BlockRec br = read_block(v, rb);
-            double fm = 0;
-            for (int cc = br.ch0; cc < br.ch1; ++cc) fm += gptr(v.freqs)[cc];
-            if (br.ch1 > br.ch0) fm /= double(br.ch1 - br.ch0);
-            ri.tscale = decorr_tscale(fm);
-            if (br.nr > 0) {
-              const int64_t mid = br.rows[br.nr / 2];
-              if (mid >= 0 && mid < v.nrow) ri.mid = int(mid);
-            }
-            if (JMODE == 2) ri.chan = (br.ch0 + br.ch1) / 2;
-          }
-          const int jrow = JMODE == 2 ? ri.mid : ri.row;
-          if (keyed && jrow >= 0) ri.key = jones_key_f(p.jp, jrow, ri.chan);
-        }
-      }
-      sRun[t] = ri;
+      sRun[t] = degrid_run<JMODE>(p, v, vrc, vblk, run_first[r0 + t], nvl, keyed);
     }
     // this lane's visibility
     bool live = k < nvl;
@@ -2217,23 +2241,267 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
       }
       __syncthreads();
     }
-    if (live) {
-      DDF_GLOBAL float2* vp = gptr_w(v.vis) + (size_t(row) * v.nchan + c) * NCORR;
-      if (NCORR == 4) {
+    if (live) degrid_residual<NCORR>(v, row, c, acc);
+  }
+}
+
+// The same pass on the matrix cores (mixed precision; the rule is at batched_quads_take).  The sum of a
+// run's visibilities over the facets is a product of (facets) x (8 real components of Y) with (facets) x
+// (cosine and sine of each visibility's phase): v_mfma_f32_4x4x1 makes an outer product per quad of
+// lanes, so a quad is four visibilities of one run (a run's last quad may be short), each lane has the
+// phasor of its own visibility (the B operand) and reads components i and i + 4 of its run's Y for
+// i = lane % 4 (the A operand; the sine's are the neighbouring lane's, with a sign), and the sums land in
+// the registers of the visibility's own lane.  Two LDS reads a lane in place of eight, and no test for a zero
+// Y: the loop, uniform over the wavefront since MFMA ignores EXEC, goes over the facets with a nonzero Y
+// anywhere in the tile.  As before the facets are summed eight at a time in FP32 fused multiply-adds
+// and then added to the FP64 sum.
+//
+// Forming Y is as much work as using it when runs are short (5 visibilities each in the case below):
+// where each antenna's Jones is in the tables is looked up once a run, neighbouring runs of one
+// Jones pair form a group whose pair is read once, and with one Stokes parameter Y is that
+// parameter times J0 S J1^H, formed once a group too.  (Groups of four or eight take registers that
+// spill: 4.10 ms and more against 3.95 with pairs.)
+// A tile is 64 quads, so at most 64 runs: the run table, Y and the rest take 38 KB where 256 runs took 56, and
+// four blocks fit a CU, all that 128 registers allow (1.0 ms of it is what surrounds the two loops, the waits
+// that the other blocks cover; with three blocks 4.4 ms; batches of 640 Y instead of 1024: 4.3).
+// 81 facets, 19.4 M visibilities in 3.1 M runs: 5.3 ms for degrid_pass_b, 3.95 here, 2.5 of it VALU issue.
+struct QuadRun {
+  double tscale;
+  uint32_t blk;     // its block (all ones: no such entry)
+  int mid;          // middle row of the block
+  uint32_t off[4];  // where its Jones are in the complex64 tables: DD, beam, each of both antennas
+};
+constexpr int kQuadY = 1024;  // (run, facet) pairs of a batch
+constexpr int kQuadGroup = 2;  // runs of a group (a power of two)
+template <int NCORR, int JMODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void degrid_pass_b_quads(
+    BatchParams p, const VisP v, const float2* M, const uint64_t* vrc, const uint32_t* vblk, const uint32_t* run_first,
+    const uint32_t* run_quad, const uint32_t* quad_run, int64_t nvl, int64_t nruns, int64_t ntile) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr int kFMax = 64;
+  constexpr int CW = NCORR == 4 ? 8 : 4;  // components of a Y: correlations 0 and 3 alone below four
+  __shared__ __attribute__((aligned(16))) float sY[kQuadY * CW];
+  __shared__ __attribute__((aligned(16))) QuadRun sRun[64];
+  __shared__ double sGeo[kFMax][3];
+  __shared__ int2 sDir[kFMax];
+  __shared__ int sLive[kFMax];
+  __shared__ int sGroup[65];  // first runs of the groups of one Jones pair, then the number of runs
+  __shared__ float sSm[32];
+  const int t = threadIdx.x, lane = t & 63, comp = t & 3;
+  const float sgn = (t & 1) ? 1.f : -1.f;
+  const JonesP& jp = p.jp;  // (its complex64 tables: batched_quads_take)
+  const bool one = p.nstokes == 1;
+  if (t < 32) sSm[t] = float(p.sm[t >> 3][(t >> 1) & 3][t & 1]);
+  for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    const int64_t r0 = quad_run[tile];
+    // lane l of each wavefront: first quad of run r0 + l within the tile
+    int rel = 64;
+    if (r0 + lane < nruns) rel = int(min(int64_t(run_quad[r0 + lane]) - tile * 64, int64_t(64)));
+    const int nr = __popcll(__ballot(rel < 64));
+    // this lane's quad, its run (the last that starts at or before it) and its visibility
+    const int quad = t >> 2;
+    int myrun = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float2 x = ld2(vp + q);
-          st2(vp + q, make_float2(float(double(x.x) - acc[q].re), float(double(x.y) - acc[q].im)));
-        }
-      } else if (NCORR == 2) {
-        const float2 x0 = ld2(vp), x1 = ld2(vp + 1);
-        st2(vp, make_float2(float(double(x0.x) - acc[0].re), float(double(x0.y) - acc[0].im)));
-        st2(vp + 1, make_float2(float(double(x1.x) - acc[3].re), float(double(x1.y) - acc[3].im)));
-      } else {
-        const float2 x0 = ld2(vp);
-        st2(vp, make_float2(float(double(x0.x) - acc[0].re), float(double(x0.y) - acc[0].im)));
-      }
+    for (int step = 32; step; step >>= 1)
+      if (__shfl(rel, myrun + step) <= quad) myrun += step;
+    const int64_t k = int64_t(run_first[r0 + myrun]) + 4 * int64_t(quad - __shfl(rel, myrun)) + comp;
+    bool live = k < (r0 + myrun + 1 < nruns ? int64_t(run_first[r0 + myrun + 1]) : nvl);
+    int64_t row = 0;
+    int c = 0;
+    if (live) {
+      const uint64_t e = vrc[k];
+      row = int64_t(uint32_t(e));
+      c = int(e >> 32);
+      live = row < v.nrow && c >= 0 && c < v.nchan;
     }
+    // uvw scaled to revolutions, as in degrid_pass_b
+    double u0 = 0, u1 = 0, u2 = 0;
+    if (live) {
+      const DDF_GLOBAL double* q = gptr(v.uvw) + 3 * row;
+      const double sc = -kPhaseScale * kInvTwoPi * gptr(v.freqs)[c];
+      u0 = q[0] * sc;
+      u1 = q[1] * sc;
+      u2 = q[2] * sc;
+    }
+    // an infinite or undefined position: its facets with a zero Y add nothing all the same
+    const bool odd = __ballot(!(fabs(u0) + fabs(u1) + fabs(u2) < INFINITY)) != 0;
+    if (t < nr) {
+      const RunInfo ri = degrid_run<JMODE>(p, v, vrc, vblk, run_first[r0 + t], nvl, JMODE != 0);
+      QuadRun qr = {ri.tscale, ri.row < 0 ? ~0u : ri.blk, ri.mid, {0, 0, 0, 0}};
+      if (JMODE != 0 && jp.pkf) {
+        qr.off[0] = prepared_offset(jp.kdims, ri.key.kt, ri.key.a0, ri.key.kc);
+        qr.off[1] = prepared_offset(jp.kdims, ri.key.kt, ri.key.a1, ri.key.kc);
+      }
+      if (JMODE != 0 && jp.pbf) {
+        qr.off[2] = prepared_offset(jp.bdims, ri.key.bt, ri.key.a0, ri.key.bc);
+        qr.off[3] = prepared_offset(jp.bdims, ri.key.bt, ri.key.a1, ri.key.bc);
+      }
+      sRun[t] = qr;
+    }
+    __syncthreads();
+    // groups: up to kQuadGroup neighbouring runs with one Jones pair
+    bool first = lane < nr;
+    if (JMODE != 0 && first && (lane & (kQuadGroup - 1))) {
+      const QuadRun& x = sRun[lane];
+      const QuadRun& y = sRun[lane - 1];
+      first = x.off[0] != y.off[0] || x.off[1] != y.off[1] || x.off[2] != y.off[2] || x.off[3] != y.off[3] ||
+              (JMODE == 2 && (x.mid < 0) != (y.mid < 0));
+    }
+    const uint64_t firsts = __ballot(first);
+    const int ng = __popcll(firsts);
+    if (t < 64 && first) sGroup[__popcll(firsts & ((uint64_t(1) << lane) - 1))] = lane;
+    if (t == 0) sGroup[ng] = nr;
+    cd acc[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    const int nrp = nr | 1;  // an odd number of Y a facet: the writes below spread over the banks
+    int fb = min(min(p.nf, kFMax), kQuadY / nrp);
+    if (fb < p.nf) fb &= ~7;
+    for (int f0 = 0; f0 < p.nf; f0 += fb) {
+      const int nfb = min(fb, p.nf - f0);
+      if (t < nfb) {
+        const FacetDev fd = gload(p.facets + f0 + t);
+        sGeo[t][0] = fd.l0;
+        sGeo[t][1] = fd.m0;
+        sGeo[t][2] = fd.n0;
+        sDir[t] = JMODE == 0 ? make_int2(0, 0)
+                             : make_int2(clampi(fd.kms_dir, 0, jp.kdims[1] - 1), clampi(fd.beam_dir, 0, jp.bdims[1] - 1));
+      }
+      if (t < kFMax) sLive[t] = 0;
+      __syncthreads();
+      // Y of every (run, facet of the batch); facets vary fastest over the threads, so the Jones
+      // loads of one run's facets (directions) are contiguous in the prepared tables
+      int grp = int(unsigned(t) / unsigned(nfb)), fi = t - grp * nfb;
+      const int dr = int(256u / unsigned(nfb)), df = 256 - dr * nfb;
+      for (; grp < ng; grp += dr, fi += df) {
+        if (fi >= nfb) {
+          fi -= nfb;
+          if (++grp >= ng) break;
+        }
+        const int ra = sGroup[grp], nrun = sGroup[grp + 1] - ra;
+        const DDF_GLOBAL float2* mf = gptr(M) + size_t(f0 + fi) * v.nblocks * p.nstokes;
+        float2 m1[kQuadGroup];  // one Stokes parameter: the values of the group's runs, read with its Jones
+        if (one) {
+#pragma unroll
+          for (int i = 0; i < kQuadGroup; ++i) {
+            m1[i] = make_float2(0.f, 0.f);
+            if (i < nrun && sRun[ra + i].blk != ~0u) m1[i] = ld2(mf + sRun[ra + i].blk);
+          }
+        }
+        M2T<float> J0, J1, K;
+        bool jones = JMODE != 0;
+        if (JMODE != 0) {
+          const QuadRun ri = sRun[ra];
+          const int2 dir = sDir[fi];
+          if (JMODE == 2) jones = ri.mid >= 0;
+          const auto entry = [&](const float2* tab, uint32_t off, int d) {
+            const DDF_GLOBAL v4f* e = reinterpret_cast<const DDF_GLOBAL v4f*>(gptr(tab)) + (size_t(off) + size_t(d)) * 2;
+            const v4f x = e[0], y = e[1];
+            return M2T<float>{{cf{x.x, x.y}, cf{x.z, x.w}, cf{y.x, y.y}, cf{y.z, y.w}}};
+          };
+          if (jp.pkf) {
+            J0 = entry(jp.pkf, ri.off[0], dir.x);
+            J1 = entry(jp.pkf, ri.off[1], dir.x);
+            if (jp.pbf) {
+              J0 = mul(J0, entry(jp.pbf, ri.off[2], dir.y));
+              J1 = mul(J1, entry(jp.pbf, ri.off[3], dir.y));
+            }
+          } else {
+            J0 = entry(jp.pbf, ri.off[2], dir.y);
+            J1 = entry(jp.pbf, ri.off[3], dir.y);
+          }
+        }
+        if (one) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) K.a[q] = cf{sSm[q * 8], sSm[q * 8 + 1]};
+          if (jones) K = mul(mul(J0, K), herm(J1));
+        }
+        bool live_f = false;
+#pragma unroll
+        for (int i = 0; i < kQuadGroup; ++i) {
+          if (i >= nrun) break;
+          const int ir = ra + i;
+          const uint32_t blk = sRun[ir].blk;
+          M2T<float> cv;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) cv.a[q] = cf{0, 0};
+          bool nz = false;
+          if (one) {
+            nz = m1[i].x != 0.f || m1[i].y != 0.f;
+            if (nz) {
+#pragma unroll
+              for (int q = 0; q < 4; ++q) cv.a[q] = K.a[q] * cf{m1[i].x, m1[i].y};
+            }
+          } else if (blk != ~0u) {
+            for (int k = 0; k < p.nstokes; ++k) {
+              const float2 x = ld2(mf + size_t(blk) * p.nstokes + k);
+              nz = nz || x.x != 0.f || x.y != 0.f;
+#pragma unroll
+              for (int q = 0; q < 4; ++q) cv.a[q] = cv.a[q] + cf{sSm[q * 8 + k * 2], sSm[q * 8 + k * 2 + 1]} * cf{x.x, x.y};
+            }
+            if (jones) cv = mul(mul(J0, cv), herm(J1));
+            if (!nz) {
+#pragma unroll
+              for (int q = 0; q < 4; ++q) cv.a[q] = cf{0, 0};
+            }
+          }
+          if (nz && p.dp.enabled && sRun[ir].mid >= 0) {
+            const FacetDev fd = gload(p.facets + f0 + fi);
+            DecorrP dp = p.dp;
+            dp.l0 = fd.dec_l0;
+            dp.m0 = fd.dec_m0;
+            const float dec = float(decorr_factor(dp, v.uvw, sRun[ir].tscale, sRun[ir].mid));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cv.a[q] = cv.a[q] * dec;
+          }
+          live_f = live_f || nz;
+          float4* yo = reinterpret_cast<float4*>(sY + (fi * nrp + ir) * CW);
+          if (NCORR == 4) {
+            yo[0] = make_float4(cv.a[0].re, cv.a[0].im, cv.a[1].re, cv.a[1].im);
+            yo[1] = make_float4(cv.a[2].re, cv.a[2].im, cv.a[3].re, cv.a[3].im);
+          } else {
+            yo[0] = make_float4(cv.a[0].re, cv.a[0].im, cv.a[3].re, cv.a[3].im);
+          }
+        }
+        if (live_f) sLive[fi] = 1;
+      }
+      __syncthreads();
+      const uint64_t facets = __ballot(sLive[lane] != 0);
+      for (int g0 = 0; g0 < nfb; g0 += 8) {
+        uint32_t todo = uint32_t(facets >> g0) & 0xFFu;
+        if (!todo) continue;
+        f4 d1 = {0.f, 0.f, 0.f, 0.f}, d2 = {0.f, 0.f, 0.f, 0.f};
+        do {
+          const int fi = g0 + __builtin_ctz(todo);
+          todo &= todo - 1;
+          const float* yp = sY + (fi * nrp + myrun) * CW + comp;
+          const float ac = yp[0], ad = CW == 8 ? yp[CW - 4] : 0.f;
+          float2 z = phasor_rev(u0 * sGeo[fi][0] + u1 * sGeo[fi][1] + u2 * sGeo[fi][2]);
+          if (odd) {
+            bool nz = false;
+            for (int q = 0; q < CW; ++q) nz = nz || yp[q - comp] != 0.f;
+            if (!nz) z = make_float2(0.f, 0.f);
+          }
+          // quad_perm [1, 0, 3, 2]: the other part of the same correlation
+          const float as = sgn * __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(ac), 0xB1, 0xF, 0xF, true));
+          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ac, z.x, d1, 0, 0, 0);
+          if (CW == 8) d2 = __builtin_amdgcn_mfma_f32_4x4x1f32(ad, z.x, d2, 0, 0, 0);
+          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(as, z.y, d1, 0, 0, 0);
+          if (CW == 8) {
+            const float at = sgn * __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(ad), 0xB1, 0xF, 0xF, true));
+            d2 = __builtin_amdgcn_mfma_f32_4x4x1f32(at, z.y, d2, 0, 0, 0);
+          }
+        } while (todo);
+        acc[0] = acc[0] + cd{d1[0], d1[1]};
+        if (CW == 8) {
+          acc[1] = acc[1] + cd{d1[2], d1[3]};
+          acc[2] = acc[2] + cd{d2[0], d2[1]};
+          acc[3] = acc[3] + cd{d2[2], d2[3]};
+        } else {
+          acc[3] = acc[3] + cd{d1[2], d1[3]};
+        }
+      }
+      __syncthreads();
+    }
+    if (live) degrid_residual<NCORR>(v, row, c, acc);
   }
 }
 
@@ -2270,13 +2538,32 @@ __global__ __launch_bounds__(256) void plan_run_flags(const BatchParams p, const
 // vrun[k] = run of visibility k (inclusive count of run starts - 1); run_first[run] = its first k.
 __global__ __launch_bounds__(256) void plan_run_ids(const int32_t* flag, const int64_t* excl, int64_t nvl,
                                                     uint32_t* vrun, uint32_t* run_first) {
+  // (either output alone)
   for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < nvl; k += int64_t(gridDim.x) * blockDim.x) {
     const int64_t r = excl[k] + flag[k] - 1;
-    vrun[k] = uint32_t(r);
-    if (flag[k]) run_first[r] = uint32_t(k);
+    if (vrun) vrun[k] = uint32_t(r);
+    if (run_first && flag[k]) run_first[r] = uint32_t(k);
   }
 }
 
+
+// Quads of four visibilities: count of each run, and (once their exclusive scan is in first) each run's
+// first quad and the run of every 64th quad.
+__global__ __launch_bounds__(256) void plan_quad_counts(const uint32_t* run_first, int64_t nruns, int64_t nvl, int32_t* cnt) {
+  for (int64_t r = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; r < nruns; r += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t end = r + 1 < nruns ? int64_t(run_first[r + 1]) : nvl;
+    cnt[r] = int32_t((end - int64_t(run_first[r]) + 3) >> 2);
+  }
+}
+
+__global__ __launch_bounds__(256) void plan_quads(const int32_t* cnt, const int64_t* first, int64_t nruns,
+                                                  uint32_t* run_quad, uint32_t* quad_run) {
+  for (int64_t r = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; r < nruns; r += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t q0 = first[r], q1 = q0 + cnt[r];
+    run_quad[r] = uint32_t(q0);
+    for (int64_t tile = (q0 + 63) >> 6; tile * 64 < q1; ++tile) quad_run[tile] = uint32_t(r);
+  }
+}
 
 // ---- adjoint of degrid pass B ------------------------------------------------------------------------
 // Forward (degrid_pass_b): vis_k = mask(corr_k * J0 (D M) J1^H) summed over facets.  Adjoint for
@@ -2705,34 +2992,49 @@ int batched_degrid_a(const BatchParams& p, const uint64_t* place, float2* M, con
 }
 
 template <int NCORR, int JMODE>
-static void launch_db_p(const BatchParams& p, const VisP& v, const float2* M, const uint64_t* vrc,
-                        const uint32_t* vblk, const uint32_t* vrun, const uint32_t* run_first, int64_t nvl, unsigned nb,
-                        hipStream_t st) {
-  if (p.prec == 1)
-    hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 1>), dim3(nb), dim3(256), 0, st, p, v, M, vrc, vblk, vrun, run_first, nvl);
+static void launch_db_p(const BatchParams& p, const VisP& v, const float2* M, const DegridRuns& d, hipStream_t st) {
+  const int64_t work = d.run_quad ? (d.nquads + 63) / 64 : (d.nvl + 255) / 256;
+  const dim3 nb(unsigned(std::min<int64_t>(work, 65536 * 4)));
+  if (d.run_quad)
+    hipLaunchKernelGGL((degrid_pass_b_quads<NCORR, JMODE>), nb, dim3(256), 0, st, p, v, M, d.vrc, d.vblk, d.run_first, d.run_quad,
+                       d.quad_run, d.nvl, d.nruns, work);
+  else if (p.prec == 1)
+    hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 1>), nb, dim3(256), 0, st, p, v, M, d.vrc, d.vblk, d.vrun, d.run_first, d.nvl);
   else if (p.prec == 2)
-    hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 2>), dim3(nb), dim3(256), 0, st, p, v, M, vrc, vblk, vrun, run_first, nvl);
+    hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 2>), nb, dim3(256), 0, st, p, v, M, d.vrc, d.vblk, d.vrun, d.run_first, d.nvl);
   else
-    hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 0>), dim3(nb), dim3(256), 0, st, p, v, M, vrc, vblk, vrun, run_first, nvl);
+    hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 0>), nb, dim3(256), 0, st, p, v, M, d.vrc, d.vblk, d.vrun, d.run_first, d.nvl);
 }
 
 template <int NCORR>
-static void launch_db_j(const BatchParams& p, const VisP& v, const float2* M, const uint64_t* vrc,
-                        const uint32_t* vblk, const uint32_t* vrun, const uint32_t* run_first, int64_t nvl, unsigned nb,
-                        hipStream_t st) {
-  if (p.jmode == 1) launch_db_p<NCORR, 1>(p, v, M, vrc, vblk, vrun, run_first, nvl, nb, st);
-  else if (p.jmode == 2) launch_db_p<NCORR, 2>(p, v, M, vrc, vblk, vrun, run_first, nvl, nb, st);
-  else launch_db_p<NCORR, 0>(p, v, M, vrc, vblk, vrun, run_first, nvl, nb, st);
+static void launch_db_j(const BatchParams& p, const VisP& v, const float2* M, const DegridRuns& d, hipStream_t st) {
+  if (p.jmode == 1) launch_db_p<NCORR, 1>(p, v, M, d, st);
+  else if (p.jmode == 2) launch_db_p<NCORR, 2>(p, v, M, d, st);
+  else launch_db_p<NCORR, 0>(p, v, M, d, st);
 }
 
-int batched_degrid_b(const BatchParams& p, const VisP& v, const float2* M, const uint64_t* vrc, const uint32_t* vblk,
-                     const uint32_t* vrun, const uint32_t* run_first, int64_t nvl, hipStream_t st) {
-  int64_t nb = (nvl + 255) / 256;
-  if (nb > 65536 * 4) nb = 65536 * 4;
-  if (nb < 1) nb = 1;
-  if (v.ncorr == 4) launch_db_j<4>(p, v, M, vrc, vblk, vrun, run_first, nvl, unsigned(nb), st);
-  else if (v.ncorr == 2) launch_db_j<2>(p, v, M, vrc, vblk, vrun, run_first, nvl, unsigned(nb), st);
-  else launch_db_j<1>(p, v, M, vrc, vblk, vrun, run_first, nvl, unsigned(nb), st);
+int batched_degrid_b(const BatchParams& p, const VisP& v, const float2* M, const DegridRuns& d, hipStream_t st) {
+  if (d.nvl < 1) return DDF_OK;
+  if (v.ncorr == 4) launch_db_j<4>(p, v, M, d, st);
+  else if (v.ncorr == 2) launch_db_j<2>(p, v, M, d, st);
+  else launch_db_j<1>(p, v, M, d, st);
+  return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
+}
+
+bool batched_quads_take(const BatchParams& p) {
+  return p.prec == 0 && (p.jmode == 0 || (!p.jp.scale && (p.jp.pkf || p.jp.pbf)));
+}
+
+static dim3 quad_grid(int64_t nruns) { return dim3(unsigned(std::min<int64_t>((nruns + 255) / 256, 65536))); }
+
+int batched_quad_counts(const DegridRuns& d, int32_t* cnt, hipStream_t st) {
+  hipLaunchKernelGGL(plan_quad_counts, quad_grid(d.nruns), dim3(256), 0, st, d.run_first, d.nruns, d.nvl, cnt);
+  return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
+}
+
+int batched_quads(const DegridRuns& d, const int32_t* cnt, const int64_t* first, uint32_t* run_quad, uint32_t* quad_run,
+                  hipStream_t st) {
+  hipLaunchKernelGGL(plan_quads, quad_grid(d.nruns), dim3(256), 0, st, cnt, first, d.nruns, run_quad, quad_run);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
 }
 

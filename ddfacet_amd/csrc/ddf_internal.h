@@ -285,9 +285,29 @@ int batched_grid_b(const BatchParams& p, const uint64_t* place, const float2* V,
 int batched_live_tiles(const BatchParams& p, const uint32_t* tile_count, uint32_t* live, hipStream_t st);
 int batched_degrid_a(const BatchParams& p, const uint64_t* place, float2* M, const BinItem* items,
                      const uint32_t* recs, uint32_t* queue, unsigned nwg, hipStream_t st);
-// vrun / run_first: the runs of the degrid visibility list (batched_run_ids)
-int batched_degrid_b(const BatchParams& p, const VisP& v, const float2* M, const uint64_t* vrc, const uint32_t* vblk,
-                     const uint32_t* vrun, const uint32_t* run_first, int64_t nvl, hipStream_t st);
+// The visibility list of degrid pass B and its runs (batched_run_ids): runs either as quads of four
+// visibilities (run_quad set: degrid_pass_b_quads) or by visibility (vrun: degrid_pass_b).
+struct DegridRuns {
+  const uint64_t* vrc = nullptr;       // row and channel of each entry
+  const uint32_t* vblk = nullptr;      // its block
+  const uint32_t* vrun = nullptr;      // its run
+  const uint32_t* run_first = nullptr; // first entry of each run
+  const uint32_t* run_quad = nullptr;  // first quad of each run
+  const uint32_t* quad_run = nullptr;  // run of every 64th quad
+  int64_t nvl = 0, nruns = 0, nquads = 0;
+};
+// Whether degrid pass B can take runs as quads: the mixed precision, and no Jones or the complex64 tables
+// (the general Jones need the registers that its four wavefronts a SIMD share).  A plan does so where a
+// quad holds at least kQuadFill visibilities on average (81 facets with Jones, 3.1 a quad: 3.95 ms, 5.3 by
+// visibility; 121 facets without, 2.5 a quad: 226 us, 359; one a quad, 1.1 M of them, 25 facets: 328 us,
+// 283), or where its tiles of 64 quads are too few for the card's 256 compute units, where tiles of
+// 256 visibilities would be fewer still (1260 visibilities, one a quad: 9.3 us, 15.9).
+bool batched_quads_take(const BatchParams& p);
+constexpr int64_t kQuadFill = 2, kQuadsFew = 64 * 256;
+int batched_degrid_b(const BatchParams& p, const VisP& v, const float2* M, const DegridRuns& d, hipStream_t st);
+int batched_quad_counts(const DegridRuns& d, int32_t* cnt, hipStream_t st);
+int batched_quads(const DegridRuns& d, const int32_t* cnt, const int64_t* first, uint32_t* run_quad, uint32_t* quad_run,
+                  hipStream_t st);
 // phase 0: run-start flags of the degrid visibility list; phase 1 (after an exclusive scan of the
 // flags into excl): the run of every visibility and the first visibility of every run
 int batched_run_ids(const BatchParams& p, const VisP& v, const uint64_t* vrc, const uint32_t* vblk, int64_t nvl,

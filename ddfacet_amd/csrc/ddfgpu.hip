@@ -1432,12 +1432,7 @@ struct ddf_plan {
   BinItem* items_d = nullptr;
   float2* V = nullptr;
   float2* M = nullptr;
-  uint64_t* vrc = nullptr;
-  uint32_t* vblk = nullptr;
-  int64_t nvl = 0;
-  uint32_t* vrun = nullptr;       // run of each degrid list entry (block and Jones key shared)
-  uint32_t* run_first = nullptr;  // first list entry of each run
-  int64_t nruns = 0;
+  DegridRuns deg = {};            // degrid visibility list: runs share a block and a Jones key
   RunList runs = {};              // grid pass A on runs (entry null: grid_pass_a)
   unsigned nwg_runs = 0;
   // work-queue counters (kQueueStride words apart): [0] grid pass A, [1, 9) grid pass B (one per item range), [9, 17) degrid
@@ -2092,37 +2087,69 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
         hipMemcpyAsync(&last_cnt, cnt + vdegrid->nblocks - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
       return bail(fail(DDF_EHIP, "copy failed"));
-    P->nvl = last_start + last_cnt;
-    P->vrc = P->alloc<uint64_t>(size_t(P->nvl));
-    P->vblk = P->alloc<uint32_t>(size_t(P->nvl));
-    if (!P->vrc || !P->vblk) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    if (batched_vlist(P->vd, vs, P->vrc, P->vblk, st)) return bail(fail(DDF_EHIP, "launch failed"));
+    DegridRuns& d = P->deg;
+    d.nvl = last_start + last_cnt;
+    uint64_t* vrc = P->alloc<uint64_t>(size_t(d.nvl));
+    uint32_t* vblk = P->alloc<uint32_t>(size_t(d.nvl));
+    if (!vrc || !vblk) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+    d.vrc = vrc;
+    d.vblk = vblk;
+    if (batched_vlist(P->vd, vs, vrc, vblk, st)) return bail(fail(DDF_EHIP, "launch failed"));
     // runs of consecutive entries with one block and one Jones key: degrid pass B forms each
     // facet's Jones product once per run
-    if (P->nvl >= (int64_t(1) << 32)) return bail(fail(DDF_EINVAL, "degrid visibility list too long for one plan"));
+    if (d.nvl >= (int64_t(1) << 32)) return bail(fail(DDF_EINVAL, "degrid visibility list too long for one plan"));
     Temp rt(st);
-    int32_t* flag = static_cast<int32_t*>(rt.get(size_t(P->nvl) * sizeof(int32_t)));
-    int64_t* excl = static_cast<int64_t*>(rt.get(size_t(P->nvl) * sizeof(int64_t)));
-    int64_t* ctmp = static_cast<int64_t*>(rt.get(size_t((P->nvl + kScanChunk - 1) / kScanChunk) * sizeof(int64_t)));
-    P->vrun = P->alloc<uint32_t>(size_t(P->nvl));
-    if (!flag || !excl || !ctmp || !P->vrun) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    if (batched_run_ids(P->pd, P->vd, P->vrc, P->vblk, P->nvl, flag, nullptr, nullptr, nullptr, 0, st))
+    int32_t* flag = static_cast<int32_t*>(rt.get(size_t(d.nvl) * sizeof(int32_t)));
+    int64_t* excl = static_cast<int64_t*>(rt.get(size_t(d.nvl) * sizeof(int64_t)));
+    int64_t* ctmp = static_cast<int64_t*>(rt.get(size_t((d.nvl + kScanChunk - 1) / kScanChunk) * sizeof(int64_t)));
+    if (!flag || !excl || !ctmp) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+    if (batched_run_ids(P->pd, P->vd, vrc, vblk, d.nvl, flag, nullptr, nullptr, nullptr, 0, st))
       return bail(fail(DDF_EHIP, "launch failed"));
-    rc = launch_scan(flag, P->nvl, 0, excl, ctmp, st);
+    // exclusive scan of n counts and the total
+    auto scan_total = [&](const int32_t* x, int64_t n, int64_t* out, int64_t* total) {
+      int rs = launch_scan(x, n, 0, out, ctmp, st);
+      if (rs) return rs;
+      int64_t last = 0;
+      int32_t own = 0;
+      if (hipMemcpyAsync(&last, out + n - 1, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
+          hipMemcpyAsync(&own, x + n - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+          hipStreamSynchronize(st) != hipSuccess)
+        return fail(DDF_EHIP, "copy failed");
+      *total = last + own;
+      return int(DDF_OK);
+    };
+    rc = scan_total(flag, d.nvl, excl, &d.nruns);
     if (rc) return bail(rc);
-    int64_t last_excl = 0;
-    int32_t last_flag = 0;
-    if (hipMemcpyAsync(&last_excl, excl + P->nvl - 1, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(&last_flag, flag + P->nvl - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-      return bail(fail(DDF_EHIP, "copy failed"));
-    P->nruns = last_excl + last_flag;
-    P->run_first = P->alloc<uint32_t>(size_t(P->nruns));
-    if (!P->run_first) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    if (batched_run_ids(P->pd, P->vd, P->vrc, P->vblk, P->nvl, flag, excl, P->vrun, P->run_first, 1, st))
+    uint32_t* run_first = P->alloc<uint32_t>(size_t(d.nruns));
+    if (!run_first) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+    d.run_first = run_first;
+    if (batched_run_ids(P->pd, P->vd, vrc, vblk, d.nvl, flag, excl, nullptr, run_first, 1, st))
       return bail(fail(DDF_EHIP, "launch failed"));
+    if (batched_quads_take(P->pd) && (d.nruns <= d.nvl / kQuadFill || d.nruns <= kQuadsFew)) {
+      int32_t* cnt4 = static_cast<int32_t*>(rt.get(size_t(d.nruns) * sizeof(int32_t)));
+      int64_t* first4 = static_cast<int64_t*>(rt.get(size_t(d.nruns) * sizeof(int64_t)));
+      if (!cnt4 || !first4) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+      if (batched_quad_counts(d, cnt4, st)) return bail(fail(DDF_EHIP, "launch failed"));
+      rc = scan_total(cnt4, d.nruns, first4, &d.nquads);
+      if (rc) return bail(rc);
+      if (d.nquads * kQuadFill <= d.nvl || d.nquads <= kQuadsFew) {
+        uint32_t* run_quad = P->alloc<uint32_t>(size_t(d.nruns));
+        uint32_t* quad_run = P->alloc<uint32_t>(size_t((d.nquads + 63) / 64));
+        if (!run_quad || !quad_run) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+        if (batched_quads(d, cnt4, first4, run_quad, quad_run, st)) return bail(fail(DDF_EHIP, "launch failed"));
+        d.run_quad = run_quad;
+        d.quad_run = quad_run;
+      }
+    }
+    if (!d.run_quad) {
+      uint32_t* vrun = P->alloc<uint32_t>(size_t(d.nvl));
+      if (!vrun) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+      d.vrun = vrun;
+      if (batched_run_ids(P->pd, P->vd, vrc, vblk, d.nvl, flag, excl, vrun, nullptr, 1, st))
+        return bail(fail(DDF_EHIP, "launch failed"));
+    }
   }
-  P->stats[4] = P->nvl;
+  P->stats[4] = P->deg.nvl;
   P->stats[6] = tile;
   P->stats[7] = G;
   int dev = 0;
@@ -2178,7 +2205,7 @@ extern "C" int ddf_plan_degrid(ddf_plan* P, float* vis, void* stream) {
     return fail(DDF_EHIP, "degrid pass A launch failed");
   P->mark(DDF_PASS_DEGRID_A, 1, st);
   P->mark(DDF_PASS_DEGRID_B, 0, st);
-  if (P->nvl && batched_degrid_b(P->pd, v, P->M, P->vrc, P->vblk, P->vrun, P->run_first, P->nvl, st))
+  if (batched_degrid_b(P->pd, v, P->M, P->deg, st))
     return fail(DDF_EHIP, "degrid pass B launch failed");
   P->mark(DDF_PASS_DEGRID_B, 1, st);
   return DDF_OK;
