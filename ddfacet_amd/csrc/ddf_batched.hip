@@ -2051,6 +2051,10 @@ __device__ __forceinline__ void degrid_residual(const VisP& v, int64_t row, int 
   }
 }
 
+// Facets of a batch: as many as leave room for the (run, facet) pairs of a tile of `nr` runs in LDS.
+constexpr int kDegridPairs = 1024, kDegridFacets = 64;
+__device__ __forceinline__ int degrid_fold(int nr, int nf) { return min(min(nf, kDegridFacets), max(1, kDegridPairs / nr)); }
+
 template <int NCORR, int JMODE, int PREC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void degrid_pass_b(BatchParams p, const VisP v, const float2* M,
                                                      const uint64_t* vrc, const uint32_t* vblk,
@@ -2059,8 +2063,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
   // Y of (run, facet) for a batch of facets, [facet][run][correlation]: as many facets per batch
   // as fit for the tile's run count (a tile of 256 visibilities holds ~20 runs with BDA, so 2
   // batches cover 81 facets; 4 facets when every visibility is a run of its own)
-  constexpr int kYCap = 4 * 256 * 4;
-  constexpr int kFMax = 64;
+  constexpr int kYCap = kDegridPairs * 4;
+  constexpr int kFMax = kDegridFacets;
   __shared__ cx<RT> sY[kYCap];
   __shared__ RunInfo sRun[256];
   // l0, m0, n0 of the batch's facets: the visibility loop reads them from LDS, not from the facet
@@ -2116,7 +2120,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
     // the sum over facets, in FP64
     cd acc[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
     __syncthreads();
-    const int FBd = min(min(p.nf, kFMax), max(1, kYCap / (4 * nr)));
+    const int FBd = degrid_fold(nr, p.nf);
     for (int f0 = 0; f0 < p.nf; f0 += FBd) {
       const int nfb = min(FBd, p.nf - f0);
       if (t < nfb) {
@@ -2174,7 +2178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
               } else {
                 jones_pair_t<RT>(jp, jrow, ri.chan, v.uvw + 3 * int64_t(jrow), p.wl_mean, J0, J1);
               }
-              cv = mul(mul(J0, cv), herm(J1));
+              cv = mul_fixed(mul_fixed(J0, cv), herm(J1));
             }
             if (p.dp.enabled && ri.mid >= 0) {
               const FacetDev fd = gload(p.facets + f);
@@ -2249,22 +2253,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
 // run's visibilities over the facets is a product of (facets) x (8 real components of Y) with (facets) x
 // (cosine and sine of each visibility's phase): v_mfma_f32_4x4x1 makes an outer product per quad of
 // lanes, so a quad is four visibilities of one run (a run's last quad may be short), each lane has the
-// phasor of its own visibility (the B operand) and reads components i and i + 4 of its run's Y for
-// i = lane % 4 (the A operand; the sine's are the neighbouring lane's, with a sign), and the sums land in
-// the registers of the visibility's own lane.  Two LDS reads a lane in place of eight, and no test for a zero
-// Y: the loop, uniform over the wavefront since MFMA ignores EXEC, goes over the facets with a nonzero Y
-// anywhere in the tile.  As before the facets are summed eight at a time in FP32 fused multiply-adds
-// and then added to the FP64 sum.
+// phasor of its own visibility (the B operand) and reads correlation lane % 4 of its run's Y (the A
+// operand), and the sums land in the registers of the visibility's own lane, real and imaginary parts in
+// one accumulator each.  One LDS read a lane in place of four, and no test for a zero Y: the loop, uniform over the
+// wavefront since MFMA ignores EXEC, goes over the facets with a nonzero Y anywhere in the tile.
+//
+// The sums are those of degrid_pass_b to the bit, so that a program's visibilities (and the FP64 loss that it
+// forms of them) do not depend on which of the two a plan takes: the same Y, the same order of the four
+// products of a part, which 4x4x1 adds as fused multiply-adds, and the same groups of facets summed in FP32
+// before they are added to the FP64 sum.  Those are eight at a time from the start of a batch of
+// degrid_pass_b, whose length follows from the runs of its tile (`fold`); the 256 visibilities of
+// a tile here lie in at most two of those, and a lane adds at the cuts of its own.
 //
 // Forming Y is as much work as using it when runs are short (5 visibilities each in the case below):
-// where each antenna's Jones is in the tables is looked up once a run, neighbouring runs of one
-// Jones pair form a group whose pair is read once, and with one Stokes parameter Y is that
-// parameter times J0 S J1^H, formed once a group too.  (Groups of four or eight take registers that
-// spill: 4.10 ms and more against 3.95 with pairs.)
+// where each antenna's Jones is in the tables is looked up once a run, and neighbouring runs of one
+// Jones pair form a group whose pair is read once.
 // A tile is 64 quads, so at most 64 runs: the run table, Y and the rest take 38 KB where 256 runs took 56, and
-// four blocks fit a CU, all that 128 registers allow (1.0 ms of it is what surrounds the two loops, the waits
-// that the other blocks cover; with three blocks 4.4 ms; batches of 640 Y instead of 1024: 4.3).
-// 81 facets, 19.4 M visibilities in 3.1 M runs: 5.3 ms for degrid_pass_b, 3.95 here, 2.5 of it VALU issue.
+// four blocks fit a CU, all that 128 registers allow: the waits of forming Y and of what surrounds the
+// loops are covered by the other blocks.
+// 81 facets, 19.4 M visibilities in 3.1 M runs: 5.3 ms for degrid_pass_b, 4.56 here (3.9 with one Stokes parameter's Y
+// formed as that parameter times a group's J0 S J1^H, which rounds otherwise).
 struct QuadRun {
   double tscale;
   uint32_t blk;     // its block (all ones: no such entry)
@@ -2276,7 +2284,7 @@ constexpr int kQuadGroup = 2;  // runs of a group (a power of two)
 template <int NCORR, int JMODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void degrid_pass_b_quads(
     BatchParams p, const VisP v, const float2* M, const uint64_t* vrc, const uint32_t* vblk, const uint32_t* run_first,
-    const uint32_t* run_quad, const uint32_t* quad_run, int64_t nvl, int64_t nruns, int64_t ntile) {
+    const uint32_t* run_quad, const uint32_t* quad_run, const uint8_t* fold, int64_t nvl, int64_t nruns, int64_t ntile) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   constexpr int kFMax = 64;
   constexpr int CW = NCORR == 4 ? 8 : 4;  // components of a Y: correlations 0 and 3 alone below four
@@ -2287,8 +2295,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
   __shared__ int sLive[kFMax];
   __shared__ int sGroup[65];  // first runs of the groups of one Jones pair, then the number of runs
   __shared__ float sSm[32];
-  const int t = threadIdx.x, lane = t & 63, comp = t & 3;
-  const float sgn = (t & 1) ? 1.f : -1.f;
+  const int t = threadIdx.x, lane = t & 63, corr = t & (CW == 8 ? 3 : 1);
   const JonesP& jp = p.jp;  // (its complex64 tables: batched_quads_take)
   const bool one = p.nstokes == 1;
   if (t < 32) sSm[t] = float(p.sm[t >> 3][(t >> 1) & 3][t & 1]);
@@ -2304,8 +2311,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
 #pragma unroll
     for (int step = 32; step; step >>= 1)
       if (__shfl(rel, myrun + step) <= quad) myrun += step;
-    const int64_t k = int64_t(run_first[r0 + myrun]) + 4 * int64_t(quad - __shfl(rel, myrun)) + comp;
+    const int64_t k = int64_t(run_first[r0 + myrun]) + 4 * int64_t(quad - __shfl(rel, myrun)) + (t & 3);
     bool live = k < (r0 + myrun + 1 < nruns ? int64_t(run_first[r0 + myrun + 1]) : nvl);
+    // the batches of degrid_pass_b: this lane's are those of the tile's first visibility or the next ones
+    const int64_t k_first = int64_t(run_first[r0]) + 4 * (tile * 64 - int64_t(run_quad[r0]));
+    const int64_t old = k_first >> 8;
+    const bool second = (k >> 8) != old;
+    const bool some_b = __ballot(live && second) != 0, some_a = __ballot(live && !second) != 0;
+    const int fold_0 = fold[old], fold_b = some_b ? fold[old + 1] : fold_0, fold_a = some_a ? fold_0 : fold_b;
     int64_t row = 0;
     int c = 0;
     if (live) {
@@ -2352,6 +2365,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
     if (t < 64 && first) sGroup[__popcll(firsts & ((uint64_t(1) << lane) - 1))] = lane;
     if (t == 0) sGroup[ng] = nr;
     cd acc[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    f4 dre = {0.f, 0.f, 0.f, 0.f}, dim_ = {0.f, 0.f, 0.f, 0.f};  // of the facets since this lane's last cut
+    bool added = false;  // whether any were added since the wavefront's last cut
     const int nrp = nr | 1;  // an odd number of Y a facet: the writes below spread over the banks
     int fb = min(min(p.nf, kFMax), kQuadY / nrp);
     if (fb < p.nf) fb &= ~7;
@@ -2386,7 +2401,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
             if (i < nrun && sRun[ra + i].blk != ~0u) m1[i] = ld2(mf + sRun[ra + i].blk);
           }
         }
-        M2T<float> J0, J1, K;
+        M2T<float> J0, J1;
         bool jones = JMODE != 0;
         if (JMODE != 0) {
           const QuadRun ri = sRun[ra];
@@ -2401,18 +2416,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
             J0 = entry(jp.pkf, ri.off[0], dir.x);
             J1 = entry(jp.pkf, ri.off[1], dir.x);
             if (jp.pbf) {
-              J0 = mul(J0, entry(jp.pbf, ri.off[2], dir.y));
-              J1 = mul(J1, entry(jp.pbf, ri.off[3], dir.y));
+              J0 = mul_fixed(J0, entry(jp.pbf, ri.off[2], dir.y));
+              J1 = mul_fixed(J1, entry(jp.pbf, ri.off[3], dir.y));
             }
           } else {
             J0 = entry(jp.pbf, ri.off[2], dir.y);
             J1 = entry(jp.pbf, ri.off[3], dir.y);
           }
-        }
-        if (one) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) K.a[q] = cf{sSm[q * 8], sSm[q * 8 + 1]};
-          if (jones) K = mul(mul(J0, K), herm(J1));
         }
         bool live_f = false;
 #pragma unroll
@@ -2424,20 +2434,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
 #pragma unroll
           for (int q = 0; q < 4; ++q) cv.a[q] = cf{0, 0};
           bool nz = false;
-          if (one) {
-            nz = m1[i].x != 0.f || m1[i].y != 0.f;
-            if (nz) {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) cv.a[q] = K.a[q] * cf{m1[i].x, m1[i].y};
-            }
-          } else if (blk != ~0u) {
-            for (int k = 0; k < p.nstokes; ++k) {
-              const float2 x = ld2(mf + size_t(blk) * p.nstokes + k);
+          if (blk != ~0u) {
+            const auto add = [&](int k, float2 x) {
               nz = nz || x.x != 0.f || x.y != 0.f;
 #pragma unroll
               for (int q = 0; q < 4; ++q) cv.a[q] = cv.a[q] + cf{sSm[q * 8 + k * 2], sSm[q * 8 + k * 2 + 1]} * cf{x.x, x.y};
-            }
-            if (jones) cv = mul(mul(J0, cv), herm(J1));
+            };
+            if (one) add(0, m1[i]);
+            else
+              for (int k = 0; k < p.nstokes; ++k) add(k, ld2(mf + size_t(blk) * p.nstokes + k));
+            if (jones) cv = mul_fixed(mul_fixed(J0, cv), herm(J1));
             if (!nz) {
 #pragma unroll
               for (int q = 0; q < 4; ++q) cv.a[q] = cf{0, 0};
@@ -2465,38 +2471,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
       }
       __syncthreads();
       const uint64_t facets = __ballot(sLive[lane] != 0);
-      for (int g0 = 0; g0 < nfb; g0 += 8) {
-        uint32_t todo = uint32_t(facets >> g0) & 0xFFu;
-        if (!todo) continue;
-        f4 d1 = {0.f, 0.f, 0.f, 0.f}, d2 = {0.f, 0.f, 0.f, 0.f};
-        do {
-          const int fi = g0 + __builtin_ctz(todo);
-          todo &= todo - 1;
-          const float* yp = sY + (fi * nrp + myrun) * CW + comp;
-          const float ac = yp[0], ad = CW == 8 ? yp[CW - 4] : 0.f;
+      // the facets after which each schedule adds its FP32 sums to the FP64 ones
+      auto cuts_of = [&](int len) {
+        const int at = (f0 + lane) % len;
+        return __ballot(lane < nfb && ((at & 7) == 7 || at == len - 1 || f0 + lane == p.nf - 1));
+      };
+      const uint64_t cut_a = cuts_of(fold_a), cut_b = fold_b == fold_a ? cut_a : cuts_of(fold_b);
+      uint64_t ends = cut_a | cut_b;
+      for (int g0 = 0; g0 < nfb;) {
+        const int g1 = ends ? __builtin_ctzll(ends) + 1 : nfb;
+        uint64_t todo = facets & (~uint64_t(0) << g0) & (~uint64_t(0) >> (64 - g1));
+        added = added || todo;
+        for (; todo; todo &= todo - 1) {
+          const int fi = __builtin_ctzll(todo);
+          const float2 y = reinterpret_cast<const float2*>(sY + (fi * nrp + myrun) * CW)[corr];
           float2 z = phasor_rev(u0 * sGeo[fi][0] + u1 * sGeo[fi][1] + u2 * sGeo[fi][2]);
           if (odd) {
+            const float* yp = sY + (fi * nrp + myrun) * CW;
             bool nz = false;
-            for (int q = 0; q < CW; ++q) nz = nz || yp[q - comp] != 0.f;
+            for (int q = 0; q < CW; ++q) nz = nz || yp[q] != 0.f;
             if (!nz) z = make_float2(0.f, 0.f);
           }
-          // quad_perm [1, 0, 3, 2]: the other part of the same correlation
-          const float as = sgn * __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(ac), 0xB1, 0xF, 0xF, true));
-          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ac, z.x, d1, 0, 0, 0);
-          if (CW == 8) d2 = __builtin_amdgcn_mfma_f32_4x4x1f32(ad, z.x, d2, 0, 0, 0);
-          d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(as, z.y, d1, 0, 0, 0);
-          if (CW == 8) {
-            const float at = sgn * __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(ad), 0xB1, 0xF, 0xF, true));
-            d2 = __builtin_amdgcn_mfma_f32_4x4x1f32(at, z.y, d2, 0, 0, 0);
+          dre = __builtin_amdgcn_mfma_f32_4x4x1f32(y.x, z.x, dre, 0, 0, 0);
+          dim_ = __builtin_amdgcn_mfma_f32_4x4x1f32(y.x, z.y, dim_, 0, 0, 0);
+          dre = __builtin_amdgcn_mfma_f32_4x4x1f32(-y.y, z.y, dre, 0, 0, 0);
+          dim_ = __builtin_amdgcn_mfma_f32_4x4x1f32(y.y, z.x, dim_, 0, 0, 0);
+        }
+        g0 = g1;
+        if (!ends) break;
+        ends &= ends - 1;
+        if (!added) continue;
+        added = !((cut_a & cut_b) >> (g1 - 1) & 1);
+        if (!added || (((second ? cut_b : cut_a) >> (g1 - 1)) & 1)) {
+#pragma unroll
+          for (int q = 0; q < (CW == 8 ? 4 : 2); ++q) {
+            acc[CW == 8 ? q : 3 * q] = acc[CW == 8 ? q : 3 * q] + cd{dre[q], dim_[q]};
+            dre[q] = dim_[q] = 0.f;
           }
-        } while (todo);
-        acc[0] = acc[0] + cd{d1[0], d1[1]};
-        if (CW == 8) {
-          acc[1] = acc[1] + cd{d1[2], d1[3]};
-          acc[2] = acc[2] + cd{d2[0], d2[1]};
-          acc[3] = acc[3] + cd{d2[2], d2[3]};
-        } else {
-          acc[3] = acc[3] + cd{d1[2], d1[3]};
         }
       }
       __syncthreads();
@@ -2562,6 +2573,15 @@ __global__ __launch_bounds__(256) void plan_quads(const int32_t* cnt, const int6
     const int64_t q0 = first[r], q1 = q0 + cnt[r];
     run_quad[r] = uint32_t(q0);
     for (int64_t tile = (q0 + 63) >> 6; tile * 64 < q1; ++tile) quad_run[tile] = uint32_t(r);
+  }
+}
+
+// Facets of a batch of degrid_pass_b for each 256 visibilities of the list: what its LDS holds of (run, facet)
+// pairs (kDegridPairs), by the tile's runs.
+__global__ __launch_bounds__(256) void plan_fold(const int32_t* flag, const int64_t* excl, int64_t nvl, int nf, uint8_t* fold) {
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i * 256 < nvl; i += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t k0 = i * 256, k1 = min(k0 + 255, nvl - 1);
+    fold[i] = uint8_t(degrid_fold(int(excl[k1] + flag[k1] - excl[k0] - flag[k0]) + 1, nf));
   }
 }
 
@@ -2997,7 +3017,7 @@ static void launch_db_p(const BatchParams& p, const VisP& v, const float2* M, co
   const dim3 nb(unsigned(std::min<int64_t>(work, 65536 * 4)));
   if (d.run_quad)
     hipLaunchKernelGGL((degrid_pass_b_quads<NCORR, JMODE>), nb, dim3(256), 0, st, p, v, M, d.vrc, d.vblk, d.run_first, d.run_quad,
-                       d.quad_run, d.nvl, d.nruns, work);
+                       d.quad_run, d.fold, d.nvl, d.nruns, work);
   else if (p.prec == 1)
     hipLaunchKernelGGL((degrid_pass_b<NCORR, JMODE, 1>), nb, dim3(256), 0, st, p, v, M, d.vrc, d.vblk, d.vrun, d.run_first, d.nvl);
   else if (p.prec == 2)
@@ -3029,6 +3049,12 @@ static dim3 quad_grid(int64_t nruns) { return dim3(unsigned(std::min<int64_t>((n
 
 int batched_quad_counts(const DegridRuns& d, int32_t* cnt, hipStream_t st) {
   hipLaunchKernelGGL(plan_quad_counts, quad_grid(d.nruns), dim3(256), 0, st, d.run_first, d.nruns, d.nvl, cnt);
+  return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
+}
+
+int batched_fold(const int32_t* flag, const int64_t* excl, int64_t nvl, int nf, uint8_t* fold, hipStream_t st) {
+  hipLaunchKernelGGL(plan_fold, dim3(unsigned(std::min<int64_t>((nvl + 65535) / 65536, 65536))), dim3(256), 0, st, flag, excl, nvl,
+                     nf, fold);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;
 }
 

@@ -101,6 +101,23 @@ __device__ __forceinline__ M2T<T> mul(const M2T<T>& x, const M2T<T>& y) {
   return M2T<T>{{x.a[0] * y.a[0] + x.a[1] * y.a[2], x.a[0] * y.a[1] + x.a[1] * y.a[3],
                  x.a[2] * y.a[0] + x.a[3] * y.a[2], x.a[2] * y.a[1] + x.a[3] * y.a[3]}};
 }
+// The same with its rounding written out (which of a part's two products a fused multiply-add takes is the
+// compiler's choice elsewhere, and differs from kernel to kernel): two kernels that form one value agree on it.
+__device__ __forceinline__ cf mul_fixed(cf a, cf b) {
+#pragma clang fp contract(off)
+  return cf{fmaf(a.re, b.re, -(a.im * b.im)), fmaf(a.im, b.re, a.re * b.im)};
+}
+__device__ __forceinline__ M2T<float> mul_fixed(const M2T<float>& x, const M2T<float>& y) {
+#pragma clang fp contract(off)
+  M2T<float> r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const cf a = mul_fixed(x.a[q & 2], y.a[q & 1]), b = mul_fixed(x.a[(q & 2) + 1], y.a[(q & 1) + 2]);
+    r.a[q] = cf{a.re + b.re, a.im + b.im};
+  }
+  return r;
+}
+__device__ __forceinline__ M2 mul_fixed(const M2& x, const M2& y) { return mul(x, y); }
 template <typename T>
 __device__ __forceinline__ M2T<T> herm(const M2T<T>& x) {
   return M2T<T>{{conj(x.a[0]), conj(x.a[2]), conj(x.a[1]), conj(x.a[3])}};
@@ -442,8 +459,8 @@ __device__ __forceinline__ void jones_pair_f(const JonesP& jp, const JonesKey& k
     J0 = prepared_jones_f(jp.pkf, jp.kdims, k.kt, k.a0, jp.kdir, k.kc);
     J1 = prepared_jones_f(jp.pkf, jp.kdims, k.kt, k.a1, jp.kdir, k.kc);
     if (jp.pbf) {
-      J0 = mul(J0, prepared_jones_f(jp.pbf, jp.bdims, k.bt, k.a0, jp.bdir, k.bc));
-      J1 = mul(J1, prepared_jones_f(jp.pbf, jp.bdims, k.bt, k.a1, jp.bdir, k.bc));
+      J0 = mul_fixed(J0, prepared_jones_f(jp.pbf, jp.bdims, k.bt, k.a0, jp.bdir, k.bc));
+      J1 = mul_fixed(J1, prepared_jones_f(jp.pbf, jp.bdims, k.bt, k.a1, jp.bdir, k.bc));
     }
   } else {
     J0 = prepared_jones_f(jp.pbf, jp.bdims, k.bt, k.a0, jp.bdir, k.bc);

@@ -294,17 +294,19 @@ struct DegridRuns {
   const uint32_t* run_first = nullptr; // first entry of each run
   const uint32_t* run_quad = nullptr;  // first quad of each run
   const uint32_t* quad_run = nullptr;  // run of every 64th quad
+  const uint8_t* fold = nullptr;       // facets of a batch of degrid_pass_b, of every 256 entries
   int64_t nvl = 0, nruns = 0, nquads = 0;
 };
 // Whether degrid pass B can take runs as quads: the mixed precision, and no Jones or the complex64 tables
 // (the general Jones need the registers that its four wavefronts a SIMD share).  A plan does so where a
-// quad holds at least kQuadFill visibilities on average (81 facets with Jones, 3.1 a quad: 3.95 ms, 5.3 by
+// quad holds at least kQuadFill visibilities on average (81 facets with Jones, 3.1 a quad: 4.56 ms, 5.3 by
 // visibility; 121 facets without, 2.5 a quad: 226 us, 359; one a quad, 1.1 M of them, 25 facets: 328 us,
 // 283), or where its tiles of 64 quads are too few for the card's 256 compute units, where tiles of
 // 256 visibilities would be fewer still (1260 visibilities, one a quad: 9.3 us, 15.9).
 bool batched_quads_take(const BatchParams& p);
 constexpr int64_t kQuadFill = 2, kQuadsFew = 64 * 256;
 int batched_degrid_b(const BatchParams& p, const VisP& v, const float2* M, const DegridRuns& d, hipStream_t st);
+int batched_fold(const int32_t* flag, const int64_t* excl, int64_t nvl, int nf, uint8_t* fold, hipStream_t st);
 int batched_quad_counts(const DegridRuns& d, int32_t* cnt, hipStream_t st);
 int batched_quads(const DegridRuns& d, const int32_t* cnt, const int64_t* first, uint32_t* run_quad, uint32_t* quad_run,
                   hipStream_t st);

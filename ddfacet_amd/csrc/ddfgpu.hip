@@ -2135,8 +2135,12 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
       if (d.nquads * kQuadFill <= d.nvl || d.nquads <= kQuadsFew) {
         uint32_t* run_quad = P->alloc<uint32_t>(size_t(d.nruns));
         uint32_t* quad_run = P->alloc<uint32_t>(size_t((d.nquads + 63) / 64));
-        if (!run_quad || !quad_run) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-        if (batched_quads(d, cnt4, first4, run_quad, quad_run, st)) return bail(fail(DDF_EHIP, "launch failed"));
+        uint8_t* fold = P->alloc<uint8_t>(size_t((d.nvl + 255) / 256));
+        if (!run_quad || !quad_run || !fold) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+        if (batched_quads(d, cnt4, first4, run_quad, quad_run, st) ||
+            batched_fold(flag, excl, d.nvl, nfacets, fold, st))
+          return bail(fail(DDF_EHIP, "launch failed"));
+        d.fold = fold;
         d.run_quad = run_quad;
         d.quad_run = quad_run;
       }
