@@ -1,6 +1,5 @@
 // Facet image side of the major cycle on gfx950: centred facet FFTs (ddf_fft.h; rocFFT for lengths
-// outside its factors or its LDS), the facet
-// normalisation image, the facet stitch and the model-to-facet extraction.
+// outside its factors or its LDS and for the facet models), the facet normalisation image, the facet stitch and the model-to-facet extraction.
 //
 //   ddf_fft2c          ModFFTW.FFTW_2Donly.fft / .ifft (DDFacet/ToolsDir/ModFFTW.py:557-600):
 //                      forward  A <- fftshift(fft2(ifftshift(A))) / N^2,
@@ -52,20 +51,34 @@ int ifail(int code, const std::string& m) {
   } while (0)
 
 // ---- centred FFTs -------------------------------------------------------------------------------
-// dst[p][y][x] = scale * src[p][(y + s) % n][(x + s) % n]
-__global__ __launch_bounds__(256) void roll2(const float2* src, float2* dst, int n, int64_t nplanes, int s,
-                                             float scale) {
-  const int64_t total = int64_t(n) * n * nplanes;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += int64_t(gridDim.x) * blockDim.x) {
-    const int64_t p = i / (int64_t(n) * n);
-    const int r = int(i - p * int64_t(n) * n);
-    const int y = r / n, x = r - (r / n) * n;
-    int ys = y + s, xs = x + s;
-    if (ys >= n) ys -= n;
-    if (xs >= n) xs -= n;
-    float2 v = src[(p * n + ys) * n + xs];
-    dst[i] = make_float2(v.x * scale, v.y * scale);
+__device__ __forceinline__ int fft_wrap(int i, int n) { return i >= n ? i - n : i; }
+
+// dst[p][y][x] = scale * src[p][(y + s) % n][(x + s) % n], a wavefront per row.
+__global__ __launch_bounds__(256) void shift_planes(const float2* src, float2* dst, int n, int64_t rows, int s,
+                                                    float scale) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t r = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6); r < rows; r += int64_t(gridDim.x) * 4) {
+    const int y = int(r % n);
+    const DDF_GLOBAL float2* in = gptr(src) + (r - y + fft_wrap(y + s, n)) * n;
+    DDF_GLOBAL float2* out = gptr_w(dst) + r * n;
+    for (int x0 = lane; x0 < n; x0 += 256) {
+      float2 v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (x0 + 64 * k < n) v[k] = ld2(in + fft_wrap(x0 + 64 * k + s, n));
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (x0 + 64 * k < n) st2(out + x0 + 64 * k, make_float2(v[k].x * scale, v[k].y * scale));
+    }
   }
+}
+
+int shift(const float2* src, float2* dst, int n, int64_t nplanes, int s, float scale, hipStream_t st) {
+  const int64_t rows = nplanes * n;
+  hipLaunchKernelGGL(shift_planes, dim3(unsigned(std::min<int64_t>((rows + 3) / 4, 1 << 20))), dim3(256), 0, st, src, dst, n,
+                     rows, s, scale);
+  HIP_OK(hipGetLastError());
+  return DDF_OK;
 }
 
 // A cached rocFFT plan is read-only once made, so calls on several streams or host threads may
@@ -76,9 +89,9 @@ struct FFTPlan {
 };
 
 std::mutex g_fft_mu;
-std::map<std::tuple<int, int64_t, int, int, int>, FFTPlan> g_fft_plans;  // (n, transforms, dir, dimensions, device)
+std::map<std::tuple<int, int64_t, int, int>, FFTPlan> g_fft_plans;  // (n, nplanes, dir, device)
 
-int get_plan(int n, int64_t ntrans, int inverse, int dims, FFTPlan** out) {
+int get_plan(int n, int64_t nplanes, int inverse, FFTPlan** out) {
   int dev = 0;
   HIP_OK(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_fft_mu);
@@ -87,7 +100,7 @@ int get_plan(int n, int64_t ntrans, int inverse, int dims, FFTPlan** out) {
     if (rocfft_setup() != rocfft_status_success) return ifail(DDF_EHIP, "rocfft_setup failed");
     setup = true;
   }
-  auto key = std::make_tuple(n, ntrans, inverse, dims, dev);
+  auto key = std::make_tuple(n, nplanes, inverse, dev);
   auto it = g_fft_plans.find(key);
   if (it != g_fft_plans.end()) {
     *out = &it->second;
@@ -97,7 +110,7 @@ int get_plan(int n, int64_t ntrans, int inverse, int dims, FFTPlan** out) {
   size_t lengths[2] = {size_t(n), size_t(n)};
   if (rocfft_plan_create(&P.plan, rocfft_placement_inplace,
                          inverse ? rocfft_transform_type_complex_inverse : rocfft_transform_type_complex_forward,
-                         rocfft_precision_single, size_t(dims), lengths, size_t(ntrans), nullptr) != rocfft_status_success)
+                         rocfft_precision_single, 2, lengths, size_t(nplanes), nullptr) != rocfft_status_success)
     return ifail(DDF_EHIP, "rocfft_plan_create failed");
   if (rocfft_plan_get_work_buffer_size(P.plan, &P.work_size) != rocfft_status_success) {
     (void)rocfft_plan_destroy(P.plan);
@@ -220,8 +233,6 @@ __global__ __launch_bounds__(256) void facet_norm_kernel(const ImgFacet* F, int 
   }
 }
 
-__device__ __forceinline__ int fft_wrap(int i, int n) { return i >= n ? i - n : i; }
-
 // Sums over the facets that cover a main-image pixel, in facet order.
 //   kStitch   Image[ch, pol, X, Y] = sum_f Im_f / FacetNorm, with Im_f[a, b] = Im[n-1-b, a] (the
 //             Im[::-1, :].T of the reference) and Im[i, j] = Re(dirty) * InvSphe * SW_grid / weights in
@@ -229,7 +240,8 @@ __device__ __forceinline__ int fft_wrap(int i, int n) { return i >= n ? i - n : 
 //   kCutAdj   adjoint of the model cut: image_bar[ch, pol, X, Y] = sum_f factor / FacetNorm[X, Y] *
 //             SW[a, b] / Sphe[a, b] * Re(plane_bar[ch, pol, n-1-b, a]), zero where Sphe < 1e-3 (the
 //             forward's flips and box read backwards).  The plane comes before the last shift of its
-//             transform and its scale: element a is at (a + shift) % n, times `scale`.
+//             transform and its scale: element (i, j) is at ((i + shift) % n, (j + shift) % n), times
+//             `scale`.
 // Bound: HBM, the real parts of the covering facets' planes (whole lines of complex values) and one
 // pass over their tapers.  A facet plane runs along X and the image along Y, so a workgroup takes 32 x
 // 32 pixels and turns each facet's tile over in LDS: both sides are read along their rows.  It first
@@ -294,7 +306,7 @@ __global__ __launch_bounds__(256) void facet_gather(const ImgFacet* F, int nf, i
         } else {
 #pragma unroll
           for (int p = 0; p < PL; ++p)
-            if (p < np) tile[p][yl][tx] = fa.model[(plane0 + p) * nn + g - a + fft_wrap(a + shift, n)].x * scale;
+            if (p < np) tile[p][yl][tx] = fa.model[(plane0 + p) * nn + size_t(fft_wrap(n - 1 - b + shift, n)) * n + fft_wrap(a + shift, n)].x * scale;
         }
       }
       if (MODE == kStitch && t < np) {
@@ -422,43 +434,6 @@ __global__ __launch_bounds__(256) void model_cut_kernel(const ImgFacet* F, int n
         const int y = y0 + ty + 8 * i, x = x0 + tx;
         if (y < n && x < n) st2(o + (size_t(p0 + p) * n + y) * n + x, make_float2(tile[p][tx][ty + 8 * i], 0.f));
       }
-    }
-    __syncthreads();
-  }
-}
-
-// dst[p][x][y] = scale src[p][(y + sy) % n][(x + sx) % n]: the transpose between the row transforms of a
-// plane, with the shifts of the centred transform, 64 x 64 elements through LDS (512-byte pieces of the rows,
-// which start off any alignment where n is odd).  Bound: HBM.  484 planes of 975^2: 1.6 ms (4.7 TB/s); 2.3 with 32 x 32.
-constexpr int kTransTile = 64;
-__global__ __launch_bounds__(256) void transpose_kernel(const float2* src, float2* dst, int n, int64_t tiles_all,
-                                                        int sy, int sx, float scale) {
-  constexpr int T = kTransTile, R = T / 4;
-  __shared__ float2 tile[T][T + 1];
-  const int tiles = (n + T - 1) / T;
-  const int tx = threadIdx.x % T, ty = threadIdx.x / T;
-  for (int64_t w = blockIdx.x; w < tiles_all; w += gridDim.x) {
-    const int64_t plane = w / (tiles * tiles);
-    const int r = int(w - plane * (tiles * tiles));
-    const int y0 = (r / tiles) * T, x0 = (r % tiles) * T;
-    const DDF_GLOBAL float2* s = gptr(src) + size_t(plane) * n * n;
-    DDF_GLOBAL float2* d = gptr_w(dst) + size_t(plane) * n * n;
-    float2 v[R];
-    const int xs = fft_wrap(x0 + tx + sx, n);
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const int y = y0 + ty + 4 * i;
-      v[i] = make_float2(0.f, 0.f);
-      if (y < n && x0 + tx < n) v[i] = ld2(s + size_t(fft_wrap(y + sy, n)) * n + xs);
-    }
-#pragma unroll
-    for (int i = 0; i < R; ++i) tile[ty + 4 * i][tx] = v[i];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const int x = x0 + ty + 4 * i, y = y0 + tx;
-      const float2 q = tile[tx][ty + 4 * i];
-      if (y < n && x < n) st2(d + size_t(x) * n + y, make_float2(q.x * scale, q.y * scale));
     }
     __syncthreads();
   }
@@ -615,8 +590,9 @@ unsigned blocks_for(int64_t n) {
   return unsigned(b);
 }
 
+// planes: where the model planes are, `per` values a facet, in place of the facets' own (null: those)
 int upload_facets(const ddf_image_facet* facets, int nf, int n, int m, hipStream_t st, ImgFacet** dout,
-                  std::vector<void*>& tmp) {
+                  std::vector<void*>& tmp, float2* planes = nullptr, int64_t per = 0) {
   std::vector<ImgFacet> h(static_cast<size_t>(nf));
   for (int i = 0; i < nf; ++i) {
     const ddf_image_facet& f = facets[i];
@@ -626,7 +602,7 @@ int upload_facets(const ddf_image_facet* facets, int nf, int n, int m, hipStream
     h[size_t(i)].inv_sphe = f.inv_sphe;
     h[size_t(i)].sw = f.sw;
     h[size_t(i)].dirty = reinterpret_cast<const float2*>(f.dirty);
-    h[size_t(i)].model = reinterpret_cast<float2*>(f.model);
+    h[size_t(i)].model = planes ? planes + i * per : reinterpret_cast<float2*>(f.model);
     h[size_t(i)].sumwt = f.sumwt;
     h[size_t(i)].sum_jones = f.sum_jones;
     const Edges& e = h[size_t(i)].e;
@@ -735,39 +711,28 @@ struct FFTCall {
   }
 };
 
-// The transforms of the facet models (forward) and of their adjoint, `per` planes of each facet: two
-// calls of rocFFT's row transform with the shifts in the transposes around them.  Forward, the cut has
-// done the first shifts and the planes end centred and scaled; the adjoint leaves its last shift, of the
-// rows, and its scale to the gather.  Both keep rocFFT: its rounding is in the predicted visibilities,
-// and a transform that rounds otherwise on one side only (the factors' constants do, by a few 1e-8 of
-// the result) would no longer be the adjoint of the other.
-static int model_transforms(const ddf_image_facet* facets, int nf, int n, int64_t per, int adjoint, hipStream_t st) {
-  bool contiguous = true;  // models[f] == models[0] + f * per planes: the transforms of every facet in one call
-  for (int f = 1; f < nf; ++f)
-    contiguous &= reinterpret_cast<float2*>(facets[f].model) == reinterpret_cast<float2*>(facets[0].model) + f * per * n * n;
-  const int groups = contiguous ? 1 : nf;
-  const int64_t nplanes = (nf / groups) * per;
-  FFTPlan* P = nullptr;
-  int rc = get_plan(n, nplanes * n, adjoint, 1, &P);
-  if (rc) return rc;
-  FFTCall call{st};
-  if ((rc = call.setup(P, nplanes * n * n))) return rc;
-  float2* t = static_cast<float2*>(call.tmp);
-  const int64_t tiles = (n + kTransTile - 1) / kTransTile, all = nplanes * tiles * tiles;
-  const dim3 g(unsigned(std::min<int64_t>(all, 1 << 20))), b(256);
-  const int in = n / 2, out = (n + 1) / 2;
-  for (int k = 0; k < groups; ++k) {
-    float2* a = reinterpret_cast<float2*>(facets[k].model);
-    if (adjoint) hipLaunchKernelGGL(transpose_kernel, g, b, 0, st, a, t, n, all, in, in, 1.f);
-    if ((rc = call.run(P, adjoint ? t : a))) return rc;
-    hipLaunchKernelGGL(transpose_kernel, g, b, 0, st, adjoint ? t : a, adjoint ? a : t, n, all, 0, out, 1.f);
-    if ((rc = call.run(P, adjoint ? a : t))) return rc;
-    if (!adjoint)
-      hipLaunchKernelGGL(transpose_kernel, g, b, 0, st, t, a, n, all, 0, out, float(1.0 / (double(n) * double(n))));
-    HIP_OK(hipGetLastError());
+// The transforms of the facet models and of their adjoint keep the 2-D rocFFT plans, one over the planes of
+// every facet where those follow one another in memory and one a facet elsewhere: their rounding is in the
+// predicted visibilities, and an FP64 loss that a program forms of those moves by some 1e-8 with another
+// transform (two 1-D plans with transposes between them round differently at 33 to 135, 243 and 343 points of
+// the odd lengths from 33 to 2025, though not at the others).
+struct ModelPlanes {
+  int groups;       // calls of the transform
+  int64_t nplanes;  // planes of one
+  FFTPlan* plan = nullptr;
+  bool joined() const { return groups == 1; }
+  float2* at(const ddf_image_facet* facets, int k) const { return reinterpret_cast<float2*>(facets[k].model); }
+  ModelPlanes(const ddf_image_facet* facets, int nf, int n, int64_t per) {
+    bool contiguous = true;
+    for (int f = 1; f < nf; ++f) contiguous &= at(facets, f) == at(facets, 0) + f * per * n * n;
+    groups = contiguous ? 1 : nf;
+    nplanes = (nf / groups) * per;
   }
-  return DDF_OK;
-}
+  int setup(FFTCall* call, int n, int inverse) {
+    int rc = get_plan(n, nplanes, inverse, &plan);
+    return rc ? rc : call->setup(plan, nplanes * n * n);
+  }
+};
 
 extern "C" int ddf_fft2c(float* planes, int32_t n, int64_t nplanes, int32_t inverse, double scale, void* stream) {
   if (!planes || n <= 0 || nplanes <= 0) return ifail(DDF_EINVAL, "bad FFT arguments");
@@ -778,7 +743,7 @@ extern "C" int ddf_fft2c(float* planes, int32_t n, int64_t nplanes, int32_t inve
   if (rc) return rc;
   if (own) return fft_planes(dims, reinterpret_cast<float2*>(planes), nplanes, inverse, scale, st);
   FFTPlan* P = nullptr;
-  rc = get_plan(n, nplanes, inverse, 2, &P);
+  rc = get_plan(n, nplanes, inverse, &P);
   if (rc) return rc;
   const int64_t total = int64_t(n) * n * nplanes;
   FFTCall call{st};
@@ -786,14 +751,10 @@ extern "C" int ddf_fft2c(float* planes, int32_t n, int64_t nplanes, int32_t inve
   float2* a = reinterpret_cast<float2*>(planes);
   float2* t = static_cast<float2*>(call.tmp);
   // ifftshift: t[j] = a[(j + n/2) % n]
-  hipLaunchKernelGGL(roll2, dim3(blocks_for(total)), dim3(256), 0, st, a, t, n, nplanes, n / 2, 1.f);
-  HIP_OK(hipGetLastError());
-  if ((rc = call.run(P, t))) return rc;
+  if ((rc = shift(a, t, n, nplanes, n / 2, 1.f, st)) || (rc = call.run(P, t))) return rc;
   // fftshift: a[k] = t[(k + (n+1)/2) % n], with the normalisation
   double norm = inverse ? scale : scale / (double(n) * double(n));
-  hipLaunchKernelGGL(roll2, dim3(blocks_for(total)), dim3(256), 0, st, t, a, n, nplanes, (n + 1) / 2, float(norm));
-  HIP_OK(hipGetLastError());
-  return DDF_OK;
+  return shift(t, a, n, nplanes, (n + 1) / 2, float(norm), st);
 }
 
 extern "C" int ddf_facet_norm(const ddf_image_facet* facets, int32_t nf, int32_t npix_facet, int32_t m,
@@ -842,12 +803,18 @@ extern "C" int ddf_model_to_grid(const ddf_image_facet* facets, int32_t nf, int3
   for (int i = 0; i < nf; ++i)
     if (!facets[i].model) return ifail(DDF_EINVAL, "facet model pointer is null");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int n = npix_facet, per = nband * npol;
+  ModelPlanes mp(facets, nf, n, per);
+  FFTCall call{st};
+  int rc = mp.setup(&call, n, 0);
+  if (rc) return rc;
+  float2* t = static_cast<float2*>(call.tmp);
   std::vector<void*> tmp;
   TmpFree guard{tmp, st};
   ImgFacet* d = nullptr;
-  int rc = upload_facets(facets, nf, npix_facet, m, st, &d, tmp);
+  // the cut goes straight to where the transform takes it
+  rc = upload_facets(facets, nf, n, m, st, &d, tmp, mp.joined() ? t : nullptr, int64_t(per) * n * n);
   if (rc) return rc;
-  const int n = npix_facet, per = nband * npol;
   int* nz = nullptr;
   HIP_OK(ddf::pool_alloc(reinterpret_cast<void**>(&nz), sizeof(int) * size_t(per) * nf, st));
   tmp.push_back(nz);
@@ -862,7 +829,14 @@ extern "C" int ddf_model_to_grid(const ddf_image_facet* facets, int32_t nf, int3
   const unsigned cuts = unsigned((n + kCutTile - 1) / kCutTile);
   hipLaunchKernelGGL(model_cut_kernel, dim3(unsigned(nf) * cuts, cuts), dim3(256), 0, st, d, n, n / 2, cut);
   HIP_OK(hipGetLastError());
-  return model_transforms(facets, nf, n, per, 0, st);
+  for (int k = 0; k < mp.groups; ++k) {
+    float2* a = mp.at(facets, k);
+    if (!mp.joined() && (rc = shift(a, t, n, mp.nplanes, 0, 1.f, st))) return rc;
+    if ((rc = call.run(mp.plan, t)) ||
+        (rc = shift(t, a, n, mp.nplanes, (n + 1) / 2, float(1.0 / (double(n) * double(n))), st)))
+      return rc;
+  }
+  return DDF_OK;
 }
 
 extern "C" int ddf_model_to_grid_adjoint(const ddf_image_facet* facets, int32_t nf, int32_t npix_facet, int32_t nband,
@@ -874,15 +848,26 @@ extern "C" int ddf_model_to_grid_adjoint(const ddf_image_facet* facets, int32_t 
     if (!facets[i].model) return ifail(DDF_EINVAL, "facet model pointer is null");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int n = npix_facet;
-  // adjoint of the forward centred FFT (1/n^2 fft): the centred inverse FFT scaled by 1/n^2
-  int rc = model_transforms(facets, nf, n, int64_t(nband) * npol, 1, st);
+  // adjoint of the forward centred FFT (1/n^2 fft): the centred inverse FFT scaled by 1/n^2; where the planes
+  // follow one another the gather takes the last shift and the scale
+  const int64_t per = int64_t(nband) * npol;
+  const float scale = float(1.0 / (double(n) * double(n)));
+  ModelPlanes mp(facets, nf, n, per);
+  FFTCall call{st};
+  int rc = mp.setup(&call, n, 1);
   if (rc) return rc;
+  float2* t = static_cast<float2*>(call.tmp);
+  for (int k = 0; k < mp.groups; ++k) {
+    float2* a = mp.at(facets, k);
+    if ((rc = shift(a, t, n, mp.nplanes, n / 2, 1.f, st)) || (rc = call.run(mp.plan, t))) return rc;
+    if (!mp.joined() && (rc = shift(t, a, n, mp.nplanes, (n + 1) / 2, scale, st))) return rc;
+  }
   std::vector<void*> tmp;
   TmpFree guard{tmp, st};
   ImgFacet* d = nullptr;
-  rc = upload_facets(facets, nf, npix_facet, m, st, &d, tmp);
+  rc = upload_facets(facets, nf, n, m, st, &d, tmp, mp.joined() ? t : nullptr, per * n * n);
   if (rc) return rc;
   const float factor = float(double(overs) * n) * float(double(overs) * n);
-  return launch_gather<kCutAdj>(d, nf, n, nband, npol, m, facet_norm, nullptr, factor, (n + 1) / 2,
-                                float(1.0 / (double(n) * double(n))), image_bar, st);
+  return launch_gather<kCutAdj>(d, nf, n, nband, npol, m, facet_norm, nullptr, factor, mp.joined() ? (n + 1) / 2 : 0,
+                                mp.joined() ? scale : 1.f, image_bar, st);
 }

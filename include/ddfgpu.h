@@ -446,8 +446,8 @@ int ddf_model_to_grid(const ddf_image_facet* facets, int32_t nf, int32_t npix_fa
                       int32_t overs, void* stream);
 
 /* Adjoint of ddf_model_to_grid (no reference counterpart; backward of the differentiable
- * forward model): takes facets[i].model as the model-grid gradient (left as work space of the adjoint
- * FFT) and writes image_bar float32 [nband][npol][m][m] (overwritten).                           */
+ * forward model): takes facets[i].model as the model-grid gradient (may be used as work space of the
+ * adjoint FFT) and writes image_bar float32 [nband][npol][m][m] (overwritten).                           */
 int ddf_model_to_grid_adjoint(const ddf_image_facet* facets, int32_t nf, int32_t npix_facet, int32_t nband,
                               int32_t npol, int32_t m, float* image_bar, const float* facet_norm,
                               int32_t overs, void* stream);
