@@ -1790,7 +1790,9 @@ __global__ __launch_bounds__(64) void grid_pass_b(BatchParams p, const uint64_t*
 // order.  No atomics; the same sum order on every run.  Workgroups take the T x T tiles that have a slot
 // in their reach (the plan's list), a lane per cell, so grids whose uv plane is mostly empty cost what
 // is in them: 121 facets x 4 bands of 975^2, 1.9 ms (3.7 with a lane for every cell of
-// every grid).  Bound: HBM (the slots are read once, the touched cells read and written).
+// every grid).  Bound: HBM (the slots are read once, the touched cells read and written), so the sum is
+// in FP64: items of a small plan hold 64 records, and the slots of a tile of 20 000 records added one after the
+// other in FP32 left an error of 6e-7 where items of 2048 records had 1e-7.
 __global__ __launch_bounds__(256) void grid_slot_reduce(BatchParams p, const float2* slots, const uint32_t* tile_first,
                                                         const uint32_t* tile_count, const uint32_t* live) {
   const int T = p.tile, h = p.halo;
@@ -1809,7 +1811,7 @@ __global__ __launch_bounds__(256) void grid_slot_reduce(BatchParams p, const flo
       const int ip = c / (T * T), r = c - ip * (T * T);
       const int y = yt + r / T, x = xt + r % T;
       if (y >= p.ny || x >= p.nx) continue;
-      float re = 0.f, im = 0.f;
+      double re = 0., im = 0.;
       const int ty0 = max(0, (y - h) / T), ty1 = min(p.ntiles_y - 1, (y + h) / T);
       const int tx0 = max(0, (x - h) / T), tx1 = min(p.ntiles_x - 1, (x + h) / T);
       for (int ty = ty0; ty <= ty1; ++ty) {
@@ -1837,10 +1839,10 @@ __global__ __launch_bounds__(256) void grid_slot_reduce(BatchParams p, const flo
           }
         }
       }
-      if (re != 0.f || im != 0.f) {
+      if (re != 0. || im != 0.) {
         DDF_GLOBAL float2* o = g + (size_t(ip) * p.ny + y) * p.nx + x;
         const float2 v = ld2(o);
-        st2(o, make_float2(v.x + re, v.y + im));
+        st2(o, make_float2(float(double(v.x) + re), float(double(v.y) + im)));
       }
     }
   }
