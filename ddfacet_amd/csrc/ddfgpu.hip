@@ -1410,7 +1410,7 @@ extern "C" int ddf_prepare_flags(uint8_t* flags, float* data, const int32_t* a0,
 // Batched plan (host side).
 // ======================================================================================================
 struct ddf_plan {
-  BatchParams pg, pd;
+  BatchParams pg, pd, pa;         // gridding, degridding, and the adjoint of degrid pass A with its own items
   VisP vg, vd;
   FacetDev* d_facets = nullptr;
   int32_t* d_support = nullptr;
@@ -1430,6 +1430,7 @@ struct ddf_plan {
   uint64_t* bstamp_d = nullptr;
   BinItem* items_g = nullptr;
   BinItem* items_d = nullptr;
+  BinItem* items_a = nullptr;
   float2* V = nullptr;
   float2* M = nullptr;
   DegridRuns deg = {};            // degrid visibility list: runs share a block and a Jones key
@@ -1561,20 +1562,138 @@ void fill_batch(BatchParams& p, const ddf_grid_desc* g, const ddf_facet* f0, con
   p.wl_mean = wl_mean;
 }
 
-// Count -> scan -> fill of the valid records, then the work items (largest first).
+// The work items of a map: of each tile's records (their counts by CF-plane group in hg) up to `chunk` an item.
+struct TileItems {
+  std::vector<BinItem> items;               // in launch order
+  std::vector<uint32_t> packs, range;       // see BatchParams
+  std::vector<int64_t> start;               // first record of each tile
+  std::vector<uint32_t> first, count;       // first slot and slots of each tile
+  int64_t records = 0;
+  int nranges = 1;
+};
+// A tile's sub-bins (CF planes) are split into ngrp groups of consecutive planes, each chunked into
+// items.  Slots are numbered tile by tile (a tile's slots consecutive, for grid_slot_reduce); the launch order
+// is (facet, band, plane group, tile), so that the workgroups running at one time read the CF planes
+// of one group and those stay in L2.
+TileItems tile_items(const BatchParams& p, std::vector<uint32_t> hg, int64_t ngrp, int chunk, int64_t light) {
+  TileItems L;
+  const int64_t ntile_fb = int64_t(p.ntiles_x) * p.ntiles_y, ntile_all = int64_t(p.nf) * p.nband * ntile_fb;
+  // A tile of up to `light` records is one item: its groups' counts go to the first group (121 facets x 4 bands:
+  // 506 000 items of 37 records otherwise, each with a tile to clear and a slot to write).
+  const int64_t whole = std::min<int64_t>(chunk, light);
+  for (int64_t i = 0; i < ntile_all; ++i) {
+    uint32_t* h = &hg[size_t(i * ngrp)];
+    int64_t all = 0;
+    for (int64_t g = 0; g < ngrp; ++g) all += h[g];
+    if (all > whole) continue;
+    std::fill(h, h + ngrp, 0u);
+    h[0] = uint32_t(all);
+  }
+  // tile-major pass: each tile's first record and first slot, each (tile, group)'s item count
+  L.start.resize(size_t(ntile_all));
+  L.first.resize(size_t(ntile_all));
+  L.count.resize(size_t(ntile_all));
+  int64_t nitem = 0;
+  for (int64_t i = 0; i < ntile_all; ++i) {
+    L.start[size_t(i)] = L.records;
+    L.first[size_t(i)] = uint32_t(nitem);
+    for (int64_t g = 0; g < ngrp; ++g) {
+      const int64_t cg = hg[size_t(i * ngrp + g)];
+      L.records += cg;
+      nitem += (cg + chunk - 1) / chunk;
+    }
+    L.count[size_t(i)] = uint32_t(nitem - L.first[size_t(i)]);
+  }
+  if (L.records >= (int64_t(1) << 32)) return L;  // (refused by the caller)
+  L.items.reserve(size_t(nitem));
+  for (int64_t fb = 0; fb < int64_t(p.nf) * p.nband; ++fb) {
+    for (int64_t g = 0; g < ngrp; ++g) {
+      for (int64_t tin = 0; tin < ntile_fb; ++tin) {
+        const int64_t i = fb * ntile_fb + tin;
+        const int64_t cg = hg[size_t(i * ngrp + g)];
+        if (cg == 0) continue;
+        int64_t g0 = 0, s0 = 0;  // records and items of the tile's earlier groups
+        for (int64_t h = 0; h < g; ++h) {
+          const int64_t ch = hg[size_t(i * ngrp + h)];
+          g0 += ch;
+          s0 += (ch + chunk - 1) / chunk;
+        }
+        for (int64_t b = 0, c = 0; b < cg; b += chunk, ++c) {
+          BinItem it;
+          it.begin = uint32_t(L.start[size_t(i)] + g0 + b);
+          it.end = uint32_t(L.start[size_t(i)] + g0 + (b + chunk < cg ? b + chunk : cg));
+          it.facet = int16_t(fb / p.nband);
+          it.band = int16_t(fb % p.nband);
+          it.tx = int16_t(tin % p.ntiles_x);
+          it.ty = int16_t(tin / p.ntiles_x);
+          it.slot = uint32_t(L.first[size_t(i)] + s0 + c);
+          L.items.push_back(it);
+        }
+      }
+    }
+  }
+  // packs of consecutive items
+  const std::vector<BinItem>& items = L.items;
+  const size_t pack_items = std::min<size_t>(kPackItems, std::max<size_t>(1, items.size() / 16384));
+  L.packs.reserve(items.size() / pack_items + 2);
+  for (size_t k = 0; k < items.size();) {
+    L.packs.push_back(uint32_t(k));
+    uint32_t n = 0;
+    for (size_t k0 = k; k < items.size() && k - k0 < pack_items && n < kPackRecords; ++k) n += items[k].end - items[k].begin;
+  }
+  const uint32_t npacks = uint32_t(L.packs.size());
+  L.packs.push_back(uint32_t(items.size()));
+  // kItemRanges contiguous ranges of the launch order with about equal record counts: the
+  // workgroups of one XCD take the packs of their own range first, so the items in flight on an
+  // XCD come from few (facet, plane group)s and their CF planes stay in that XCD's L2.  Only with
+  // many items: with few, the heaviest items (neighbouring uv tiles) would share one XCD's CUs, so
+  // all items then form one range.
+  L.nranges = items.size() >= kRangeMinItems ? kItemRanges : 1;
+  L.range.assign(size_t(L.nranges) + 1, npacks);
+  L.range[0] = 0;
+  if (L.nranges > 1) {
+    int64_t acc = 0;
+    int x = 1;
+    for (uint32_t k = 0; k < npacks && x < L.nranges; ++k) {
+      for (uint32_t i = L.packs[k]; i < L.packs[k + 1]; ++i) acc += int64_t(items[i].end) - items[i].begin;
+      while (x < L.nranges && acc * L.nranges >= L.records * x) L.range[size_t(x++)] = k + 1;
+    }
+  }
+  return L;
+}
+
+// The items, packs and ranges on the device, and what of them the passes read from p.
+int upload_items(ddf_plan* P, BatchParams& p, const TileItems& L, BinItem** items_out, hipStream_t st) {
+  BinItem* d_items = P->alloc<BinItem>(L.items.size());
+  uint32_t* d_range = P->alloc<uint32_t>(L.range.size());
+  uint32_t* d_packs = P->alloc<uint32_t>(L.packs.size());
+  if (!d_items || !d_range || !d_packs) return fail(DDF_ENOMEM, "plan allocation failed");
+  if (!L.items.empty())
+    HIP_TRY(hipMemcpyAsync(d_items, L.items.data(), L.items.size() * sizeof(BinItem), hipMemcpyHostToDevice, st));
+  HIP_TRY(hipMemcpyAsync(d_range, L.range.data(), L.range.size() * 4, hipMemcpyHostToDevice, st));
+  HIP_TRY(hipMemcpyAsync(d_packs, L.packs.data(), L.packs.size() * 4, hipMemcpyHostToDevice, st));
+  p.pack_range = d_range;
+  p.pack_first = d_packs;
+  p.npacks = uint32_t(L.packs.size()) - 1;
+  p.nranges = L.nranges;
+  p.nitems_b = uint32_t(L.items.size());
+  // degrid pass A: a workgroup of one wavefront where an item has few records for four
+  p.tile_threads = L.records < int64_t(L.items.size()) * 192 ? 64 : 256;
+  *items_out = d_items;
+  return DDF_OK;
+}
+
+// Count -> scan -> fill of the valid records, then the work items (largest first).  adj: the items of
+// the adjoint pass over the same records (null: none).
 int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place, int chunk, uint32_t** recs_out,
-               BinItem** items_out, uint32_t* nitems, int64_t* nrec, bool stamp_order,
-               hipStream_t st, uint32_t** tile_first_out = nullptr, uint32_t** tile_count_out = nullptr) {
+               BinItem** items_out, int64_t* nrec, bool stamp_order, hipStream_t st, uint32_t** tile_first_out,
+               uint32_t** tile_count_out, BatchParams* adj, BinItem** adj_items_out) {
   const int64_t nsub = 2 * int64_t(p.nw);  // CF-plane sub-bins of each tile
   const int64_t ntile_all = int64_t(p.nf) * p.nband * p.ntiles_y * p.ntiles_x;
   const int64_t nbins = ntile_all * nsub;
   uint32_t* counts = P->alloc<uint32_t>(size_t(nbins));
   uint32_t* fill = P->alloc<uint32_t>(size_t(nbins));
   int64_t* bstart = P->alloc<int64_t>(size_t(nbins));
-  // A tile's sub-bins (CF planes) are split into ngrp groups of consecutive planes, each chunked
-  // into items.  Slots are numbered tile by tile (a tile's slots consecutive, for
-  // grid_slot_reduce); the launch order is (facet, band, plane group, tile), so that the
-  // workgroups running at one time read the CF planes of one group and those stay in L2.
   const int64_t ngrp = nsub < 4 ? nsub : 4;
   uint32_t* gcount = P->alloc<uint32_t>(size_t(ntile_all * ngrp));
   int64_t* tstart = P->alloc<int64_t>(size_t(ntile_all));
@@ -1591,122 +1710,52 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
   // Records of an item: those asked for, or 2048, down to 64 where a plan has too few to give every
   // wavefront of the tile passes an item (9 facets of 189^2, 11 000 records: a wavefront with a heavy
   // tile's 1000 records took longer than all others together).
+  const int most = chunk > 0 ? chunk : 2048;
   if (chunk <= 0) {
     int64_t all = 0;
     for (uint32_t c : hg) all += c;
-    chunk = int(std::min<int64_t>(2048, std::max<int64_t>(64, all / 4096 / 64 * 64)));
+    chunk = int(std::min<int64_t>(most, std::max<int64_t>(64, all / 4096 / 64 * 64)));
   }
-  // A light tile is one item: its groups' counts go to the first group (121 facets x 4 bands: 506 000
-  // items of 37 records otherwise, each with a tile to clear and a slot to write).
-  const int64_t whole = std::min<int64_t>(chunk, kWholeTileRecords);
-  for (int64_t i = 0; i < ntile_all; ++i) {
-    uint32_t* h = &hg[size_t(i * ngrp)];
-    int64_t all = 0;
-    for (int64_t g = 0; g < ngrp; ++g) all += h[g];
-    if (all > whole) continue;
-    std::fill(h, h + ngrp, 0u);
-    h[0] = uint32_t(all);
-  }
-  // tile-major pass: each tile's first record and first slot, each (tile, group)'s item count
-  std::vector<int64_t> ts(static_cast<size_t>(ntile_all));
-  std::vector<uint32_t> tfirst(static_cast<size_t>(ntile_all)), tcount(static_cast<size_t>(ntile_all));
-  int64_t tot = 0, nitem = 0;
-  for (int64_t i = 0; i < ntile_all; ++i) {
-    ts[size_t(i)] = tot;
-    tfirst[size_t(i)] = uint32_t(nitem);
-    for (int64_t g = 0; g < ngrp; ++g) {
-      const int64_t cg = hg[size_t(i * ngrp + g)];
-      tot += cg;
-      nitem += (cg + chunk - 1) / chunk;
-    }
-    tcount[size_t(i)] = uint32_t(nitem - tfirst[size_t(i)]);
-  }
+  const TileItems L = tile_items(p, hg, ngrp, chunk, kWholeTileRecords);
+  const int64_t tot = L.records;
   if (tot >= (int64_t(1) << 32)) return fail(DDF_EINVAL, "too many (block, facet) records for one plan");
-  // items in launch order
-  std::vector<BinItem> items;
-  items.reserve(size_t(nitem));
-  const int64_t ntile_fb = int64_t(p.ntiles_x) * p.ntiles_y;
-  for (int64_t fb = 0; fb < int64_t(p.nf) * p.nband; ++fb) {
-    for (int64_t g = 0; g < ngrp; ++g) {
-      for (int64_t tin = 0; tin < ntile_fb; ++tin) {
-        const int64_t i = fb * ntile_fb + tin;
-        int64_t g0 = 0, s0 = 0;  // records and items of the tile's earlier groups
-        for (int64_t h = 0; h < g; ++h) {
-          const int64_t ch = hg[size_t(i * ngrp + h)];
-          g0 += ch;
-          s0 += (ch + chunk - 1) / chunk;
-        }
-        const int64_t cg = hg[size_t(i * ngrp + g)];
-        for (int64_t b = 0, c = 0; b < cg; b += chunk, ++c) {
-          BinItem it;
-          it.begin = uint32_t(ts[size_t(i)] + g0 + b);
-          it.end = uint32_t(ts[size_t(i)] + g0 + (b + chunk < cg ? b + chunk : cg));
-          it.facet = int16_t(fb / p.nband);
-          it.band = int16_t(fb % p.nband);
-          it.tx = int16_t(tin % p.ntiles_x);
-          it.ty = int16_t(tin / p.ntiles_x);
-          it.slot = uint32_t(tfirst[size_t(i)] + s0 + c);
-          items.push_back(it);
-        }
-      }
-    }
-  }
-  HIP_TRY(hipMemcpyAsync(tstart, ts.data(), ts.size() * 8, hipMemcpyHostToDevice, st));
+  HIP_TRY(hipMemcpyAsync(tstart, L.start.data(), L.start.size() * 8, hipMemcpyHostToDevice, st));
   if (batched_bin_starts(counts, tstart, ntile_all, int(nsub), bstart, st))
     return fail(DDF_EHIP, "plan_bin_starts launch failed");
-  // packs of consecutive items
-  const size_t pack_items = std::min<size_t>(kPackItems, std::max<size_t>(1, items.size() / 16384));
-  std::vector<uint32_t> packs;
-  packs.reserve(items.size() / pack_items + 2);
-  for (size_t k = 0; k < items.size();) {
-    packs.push_back(uint32_t(k));
-    uint32_t n = 0;
-    for (size_t k0 = k; k < items.size() && k - k0 < pack_items && n < kPackRecords; ++k) n += items[k].end - items[k].begin;
-  }
-  const uint32_t npacks = uint32_t(packs.size());
-  packs.push_back(uint32_t(items.size()));
-  // kItemRanges contiguous ranges of the launch order with about equal record counts: the
-  // workgroups of one XCD take the packs of their own range first, so the items in flight on an
-  // XCD come from few (facet, plane group)s and their CF planes stay in that XCD's L2.  Only with
-  // many items: with few, the heaviest items (neighbouring uv tiles) would share one XCD's CUs, so
-  // all items then form one range.
-  const int nranges = items.size() >= kRangeMinItems ? kItemRanges : 1;
-  std::vector<uint32_t> range(size_t(nranges) + 1, npacks);
-  range[0] = 0;
-  if (nranges > 1) {
-    int64_t acc = 0;
-    int x = 1;
-    for (uint32_t k = 0; k < npacks && x < nranges; ++k) {
-      for (uint32_t i = packs[k]; i < packs[k + 1]; ++i) acc += int64_t(items[i].end) - items[i].begin;
-      while (x < nranges && acc * nranges >= tot * x) range[size_t(x++)] = k + 1;
-    }
-  }
   uint32_t* recs = P->alloc<uint32_t>(size_t(tot));
-  BinItem* d_items = P->alloc<BinItem>(items.size());
-  uint32_t* d_range = P->alloc<uint32_t>(range.size());
-  uint32_t* d_packs = P->alloc<uint32_t>(packs.size());
-  if (!recs || !d_items || !d_range || !d_packs) return fail(DDF_ENOMEM, "plan allocation failed");
-  if (!items.empty())
-    HIP_TRY(hipMemcpyAsync(d_items, items.data(), items.size() * sizeof(BinItem), hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d_range, range.data(), range.size() * 4, hipMemcpyHostToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d_packs, packs.data(), packs.size() * 4, hipMemcpyHostToDevice, st));
-  p.pack_range = d_range;
-  p.pack_first = d_packs;
-  p.npacks = npacks;
-  p.nranges = nranges;
-  // degrid pass A: a workgroup of one wavefront where an item has few records for four
-  p.tile_threads = tot < int64_t(items.size()) * 192 ? 64 : 256;
+  if (!recs) return fail(DDF_ENOMEM, "plan allocation failed");
+  BinItem* d_items = nullptr;
+  int rc = upload_items(P, p, L, &d_items, st);
+  if (rc) return rc;
   if (tile_first_out) {
     uint32_t* tf = P->alloc<uint32_t>(size_t(ntile_all));
     uint32_t* tc = P->alloc<uint32_t>(size_t(ntile_all));
     if (!tf || !tc) return fail(DDF_ENOMEM, "plan allocation failed");
-    HIP_TRY(hipMemcpyAsync(tf, tfirst.data(), size_t(ntile_all) * 4, hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(tc, tcount.data(), size_t(ntile_all) * 4, hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(tf, L.first.data(), size_t(ntile_all) * 4, hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(tc, L.count.data(), size_t(ntile_all) * 4, hipMemcpyHostToDevice, st));
     *tile_first_out = tf;
     *tile_count_out = tc;
   }
   if (batched_fill(p, v.nblocks, place, bstart, fill, recs, st)) return fail(DDF_EHIP, "plan_fill launch failed");
-  if (batched_sort_items(p, place, recs, tot, d_items, uint32_t(items.size()), stamp_order, st))
+  // the records are sorted within the larger items; where the adjoint has items of its own, the others
+  // are parts of them
+  BinItem* sort_items = d_items;
+  uint32_t nsort = p.nitems_b;
+  TileItems A;
+  if (adj) {
+    // The adjoint adds in FP32 both in an item's tile and, by atomics, in the grids: a cell's error grows with
+    // the items of its tile (with 64 records each the gradients of dense small plans came out three times as far
+    // from 64 bits) and with the records of an item (tiles of 512 records taken whole: 1.4 times).  So its items
+    // are a plane group's 2048 records: 25 facets x 4 bands, 5.64 ms a gradient, 5.61 with tiles taken
+    // whole, 6.00 with FP64 tiles.
+    *adj = p;
+    A = tile_items(p, hg, ngrp, most, 0);
+    rc = upload_items(P, *adj, A, adj_items_out, st);
+    if (rc) return rc;
+    sort_items = *adj_items_out;
+    nsort = adj->nitems_b;
+  }
+  if (batched_sort_items(p, place, recs, tot, sort_items, nsort, stamp_order, st))
     return fail(DDF_EHIP, "sorting the records of the work items failed");
   HIP_TRY(hipStreamSynchronize(st));
   // the binning buffers are not needed by the cycle
@@ -1717,7 +1766,6 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
   P->release(tstart, size_t(ntile_all));
   *recs_out = recs;
   *items_out = d_items;
-  *nitems = uint32_t(items.size());
   *nrec = tot;
   return DDF_OK;
 }
@@ -1961,11 +2009,11 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   if (vgrid->nblocks && batched_place(P->pg, P->vg, false, P->place_g, st)) return bail(fail(DDF_EHIP, "plan_place failed"));
   if (vdegrid->nblocks && batched_place(P->pd, P->vd, true, P->place_d, st)) return bail(fail(DDF_EHIP, "plan_place failed"));
   // bins
-  uint32_t ni = 0;
   int64_t nr = 0;
-  rc = build_bins(P, P->pg, P->vg, P->place_g, chunk, &P->recs_g, &P->items_g, &ni, &nr, true, st, &P->tile_first_g, &P->tile_count_g);
+  rc = build_bins(P, P->pg, P->vg, P->place_g, chunk, &P->recs_g, &P->items_g, &nr, true, st, &P->tile_first_g, &P->tile_count_g,
+                  nullptr, nullptr);
   if (rc) return bail(rc);
-  P->pg.nitems_b = ni;
+  const uint32_t ni = P->pg.nitems_b;
   P->stats[0] = nr;
   P->stats[2] = ni;
   P->bstamp_g = P->alloc<uint64_t>(size_t(nr));
@@ -1995,11 +2043,10 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
         return bail(fail(DDF_ENOMEM, "plan allocation failed"));
     }
   }
-  rc = build_bins(P, P->pd, P->vd, P->place_d, chunk, &P->recs_d, &P->items_d, &ni, &nr, false, st);
+  rc = build_bins(P, P->pd, P->vd, P->place_d, chunk, &P->recs_d, &P->items_d, &nr, false, st, nullptr, nullptr, &P->pa, &P->items_a);
   if (rc) return bail(rc);
-  P->pd.nitems_b = ni;
   P->stats[1] = nr;
-  P->stats[3] = ni;
+  P->stats[3] = P->pd.nitems_b;
   P->bstamp_d = P->alloc<uint64_t>(size_t(nr));
   if (!P->bstamp_d || batched_stamp_records(P->pd, P->place_d, P->recs_d, nr, P->bstamp_d, st))
     return bail(fail(DDF_ENOMEM, "plan allocation failed"));
@@ -2226,7 +2273,7 @@ extern "C" int ddf_plan_degrid_adjoint(ddf_plan* P, const float* vis_bar, void* 
     return fail(DDF_EHIP, "degrid adjoint pass B launch failed");
   P->mark(DDF_PASS_ADJ_B, 1, st);
   P->mark(DDF_PASS_ADJ_A, 0, st);
-  if (P->pd.nitems_b && batched_degrid_a_adjoint(P->pd, P->bstamp_d, P->M, P->items_d, P->recs_d, P->queue(2 + 2 * kItemRanges), P->nwg_tiles[2], st))
+  if (P->pa.nitems_b && batched_degrid_a_adjoint(P->pa, P->bstamp_d, P->M, P->items_a, P->recs_d, P->queue(2 + 2 * kItemRanges), P->nwg_tiles[2], st))
     return fail(DDF_EHIP, "degrid adjoint pass A launch failed");
   P->mark(DDF_PASS_ADJ_A, 1, st);
   return DDF_OK;
