@@ -464,8 +464,8 @@ __global__ __launch_bounds__(256) void model_nonzero_kernel(const ImgFacet* F, i
 // in place: the shifts of the centred transform are index offsets of a pass's loads and stores and the
 // scale is applied by the last store.  Bound: HBM; a strip of C columns holds n C values in LDS, C such
 // that two workgroups share a CU, and is read in C * 8-byte pieces.  Loads are issued eight at a time
-// before their LDS stores.  484 planes of 975^2 (3.7 GB each way): columns 2.8 ms, rows 2.1 ms; with one
-// load at a time 4.0 and 3.5; the rocFFT plan with its transposes and the shifts around it 9.1 together.
+// before their LDS stores.  484 planes of 975^2 (3.7 GB each way): columns 3.0 ms, rows 2.5 ms; the
+// rocFFT plan with its transposes and the shifts around it 9.1 together.
 struct FftPass {
   int shift_in, shift_out;  // element j takes source (j + shift_in) % n; result p is frequency (p + shift_out) % n
   int inverse;
