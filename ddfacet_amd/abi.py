@@ -228,6 +228,7 @@ EXTRA_SIGNATURES = {
     "ddf_plan_timing": [C.c_void_p, C.c_int32],
     "ddf_plan_pass_ms": [C.c_void_p, C.POINTER(C.c_float), C.c_int32],
     "ddf_plan_destroy": [C.c_void_p],
+    "ddf_trim_memory": [],
     "ddf_plan_degrid_adjoint": [C.c_void_p, C.c_void_p, C.c_void_p],
     "ddf_model_to_grid_adjoint": [C.POINTER(ddf_image_facet), C.c_int32, C.c_int32, C.c_int32, C.c_int32,
                                   C.c_int32, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p],

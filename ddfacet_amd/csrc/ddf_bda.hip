@@ -339,10 +339,7 @@ struct ddf_bda_builder {
   int64_t* seg = nullptr;
   int64_t* blk_off = nullptr;
   int64_t* word_off = nullptr;
-  ~ddf_bda_builder() {
-    if (!arena.empty()) (void)hipDeviceSynchronize();
-    arena.release_all(nullptr);
-  }
+  ~ddf_bda_builder() { arena.close(); }
   template <typename T>
   T* alloc(size_t n) {
     return static_cast<T*>(arena.get(std::max<size_t>(n, 1) * sizeof(T), st));

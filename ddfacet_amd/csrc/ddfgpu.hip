@@ -895,41 +895,53 @@ int launch_degrid_r(const KParams& p, int jmode, int lg, unsigned nb, hipStream_
 namespace ddf {
 void set_last_error(const std::string& msg) { g_err = msg; }
 
-hipError_t pool_alloc(void** p, size_t bytes, hipStream_t st) {
+// The current device's pool, made at its first use (0: this one has none).
+static hipError_t device_pool(hipMemPool_t* pool) {
   static std::mutex mu;
   static hipMemPool_t pools[64] = {};
+  *pool = nullptr;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= 64) return hipMallocAsync(p, bytes, st);
-  hipMemPool_t pool;
-  {
-    std::lock_guard<std::mutex> lk(mu);
-    if (!pools[dev]) {
-      hipMemPoolProps props;
-      std::memset(&props, 0, sizeof(props));
-      props.allocType = hipMemAllocationTypePinned;
-      props.location.type = hipMemLocationTypeDevice;
-      props.location.id = dev;
-      hipMemPool_t made = nullptr;
-      e = hipMemPoolCreate(&made, &props);
-      if (e != hipSuccess) return e;
-      uint64_t keep = kPoolKeep;
-      e = hipMemPoolSetAttribute(made, hipMemPoolAttrReleaseThreshold, &keep);
-      if (e != hipSuccess) {
-        (void)hipMemPoolDestroy(made);
-        return e;
-      }
-      pools[dev] = made;
+  if (e != hipSuccess || dev < 0 || dev >= 64) return e;
+  std::lock_guard<std::mutex> lk(mu);
+  if (!pools[dev]) {
+    hipMemPoolProps props;
+    std::memset(&props, 0, sizeof(props));
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    hipMemPool_t made = nullptr;
+    e = hipMemPoolCreate(&made, &props);
+    if (e != hipSuccess) return e;
+    uint64_t keep = kPoolKeep;
+    e = hipMemPoolSetAttribute(made, hipMemPoolAttrReleaseThreshold, &keep);
+    if (e != hipSuccess) {
+      (void)hipMemPoolDestroy(made);
+      return e;
     }
-    pool = pools[dev];
+    pools[dev] = made;
   }
+  *pool = pools[dev];
+  return hipSuccess;
+}
+
+hipError_t pool_alloc(void** p, size_t bytes, hipStream_t st) {
+  hipMemPool_t pool;
+  hipError_t e = device_pool(&pool);
+  if (e != hipSuccess) return e;
+  if (!pool) return hipMallocAsync(p, bytes, st);
   e = hipMallocFromPoolAsync(p, bytes, pool, st);
   if (e == hipSuccess) return e;
   (void)hipGetLastError();
   (void)hipStreamSynchronize(st);
   (void)hipMemPoolTrimTo(pool, 0);
   return hipMallocFromPoolAsync(p, bytes, pool, st);
+}
+
+hipError_t pool_trim(size_t keep) {
+  hipMemPool_t pool;
+  const hipError_t e = device_pool(&pool);
+  return e != hipSuccess || !pool ? e : hipMemPoolTrimTo(pool, keep);
 }
 }  // namespace ddf
 
@@ -1455,9 +1467,7 @@ struct ddf_plan {
   hipEvent_t ev[DDF_PLAN_NPASS][2] = {};
   int ev_set[DDF_PLAN_NPASS] = {};
   ~ddf_plan() {
-    // a cycle may still be under way on any stream
-    if (!arena.empty()) (void)hipDeviceSynchronize();
-    arena.release_all(nullptr);
+    arena.close();  // (a cycle may still be under way on any stream)
     for (auto& e : ev)
       for (hipEvent_t x : e)
         if (x) (void)hipEventDestroy(x);
@@ -2317,6 +2327,12 @@ extern "C" int ddf_plan_pass_ms(ddf_plan* P, float* ms, int32_t n) {
     HIP_TRY(hipEventSynchronize(P->ev[i][1]));
     HIP_TRY(hipEventElapsedTime(&ms[i], P->ev[i][0], P->ev[i][1]));
   }
+  return DDF_OK;
+}
+
+extern "C" int ddf_trim_memory(void) {
+  HIP_TRY(hipDeviceSynchronize());
+  HIP_TRY(pool_trim(0));
   return DDF_OK;
 }
 

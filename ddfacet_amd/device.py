@@ -6,6 +6,8 @@ addresses to ``marshal.fill_structs`` and keeps them alive for the duration of a
 import numpy as np
 import torch
 
+from ._lib import check, lib
+
 _BOOL_AS = np.uint8
 
 
@@ -31,6 +33,12 @@ def to_device(a, device):
     if a.dtype == np.bool_:
         a = a.view(_BOOL_AS)
     return torch.from_numpy(a).to(device, non_blocking=False)
+
+
+def trim_memory(device=None):
+    """Return the freed device memory that the library keeps for its next calls (at most 4 GiB) to the device."""
+    with torch.cuda.device(device if device is not None else torch.cuda.current_device()):
+        check(lib().ddf_trim_memory())
 
 
 class Staging:

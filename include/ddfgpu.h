@@ -287,6 +287,10 @@ int ddf_plan_timing(ddf_plan* plan, int32_t enable);
 int ddf_plan_pass_ms(ddf_plan* plan, float* ms, int32_t n);
 int ddf_plan_destroy(ddf_plan* plan);
 
+/* Freed buffers stay with the library for its next calls, up to 4 GiB a device; this returns those of the
+ * current device (for another allocator of the process that needs the memory).  Waits for the device. */
+int ddf_trim_memory(void);
+
 /* ---- chunk staging --------------------------------------------------------------------------
  * The baseline-time sort of ClassMS.ReadData (DDFacet/Data/ClassMS.py:575-586):
  * index[k] = the row of rank k in sorted(zip(A0, A1, TIME, range(nrow))) (antennas < 65536).
