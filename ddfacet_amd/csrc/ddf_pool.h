@@ -31,6 +31,7 @@ class PoolArena {
       void* p = nullptr;
       if (pool_alloc(&p, own ? bytes : slab, st) != hipSuccess) return nullptr;
       (own ? own_ : slabs_).push_back(p);
+      bytes_ += own ? bytes : slab;
       if (own) return p;
       cur_ = static_cast<char*>(p);
       left_ = slab;
@@ -40,21 +41,15 @@ class PoolArena {
     left_ -= bytes;
     return p;
   }
-  // gives back a buffer that has an allocation of its own (one cut from a slab goes with the slab)
-  void release(void* p, hipStream_t st) {
-    auto it = std::find(own_.begin(), own_.end(), p);
-    if (it == own_.end()) return;
-    (void)hipFreeAsync(p, st);
-    own_.erase(it);
-  }
   void release_all(hipStream_t st) {
     for (void* p : own_) (void)hipFreeAsync(p, st);
     for (void* p : slabs_) (void)hipFreeAsync(p, st);
     own_.clear();
     slabs_.clear();
     cur_ = nullptr;
-    left_ = 0;
+    left_ = bytes_ = 0;
   }
+  size_t bytes() const { return bytes_; }  // of device memory held
   bool empty() const { return own_.empty() && slabs_.empty(); }
   // Gives everything back at the end of an object whose work may still run on any stream: waits for the device of
   // the buffers, whichever one is current, and hands what the pool does not keep to the device before it returns.
@@ -74,7 +69,7 @@ class PoolArena {
   int dev_ = 0;  // of the buffers
   std::vector<void*> own_, slabs_;
   char* cur_ = nullptr;  // of the newest slab
-  size_t left_ = 0;
+  size_t left_ = 0, bytes_ = 0;
 };
 
 }  // namespace ddf

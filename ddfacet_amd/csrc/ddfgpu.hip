@@ -796,7 +796,10 @@ struct Temp {
   PoolArena arena;
   explicit Temp(hipStream_t s) : st(s) {}
   void* get(size_t bytes) { return arena.get(bytes, st); }
-  ~Temp() { arena.release_all(st); }
+  template <typename T>
+  T* get(size_t n) { return static_cast<T*>(arena.get(n * sizeof(T), st)); }
+  void free() { arena.release_all(st); }
+  ~Temp() { free(); }
 };
 
 int resolve_block_index(const ddf_vis* v, Temp& tmp, const int64_t** out) {
@@ -1426,9 +1429,6 @@ struct ddf_plan {
   VisP vg, vd;
   FacetDev* d_facets = nullptr;
   int32_t* d_support = nullptr;
-  // placement records of both maps while the plan is built (ddf_plan_placements recomputes them)
-  uint64_t* place_g = nullptr;
-  uint64_t* place_d = nullptr;
   // pair codes (0x80 | band for a placed (block, facet) record) read by the cycle passes
   uint8_t* pcode_g = nullptr;
   uint8_t* pcode_d = nullptr;
@@ -1479,17 +1479,7 @@ struct ddf_plan {
   }
   template <typename T>
   T* alloc(size_t n) {
-    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-    void* p = arena.get(bytes, st);
-    if (p) stats[5] += int64_t(bytes);
-    return static_cast<T*>(p);
-  }
-  // frees one allocation of this plan (bytes as allocated) once the stream of the build is through with it
-  template <typename T>
-  void release(T*& p, size_t n) {
-    arena.release(p, st);
-    stats[5] -= int64_t(std::max<size_t>(n, 1) * sizeof(T));
-    p = nullptr;
+    return static_cast<T*>(arena.get(std::max<size_t>(n, 1) * sizeof(T), st));
   }
 };
 
@@ -1701,12 +1691,13 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
   const int64_t nsub = 2 * int64_t(p.nw);  // CF-plane sub-bins of each tile
   const int64_t ntile_all = int64_t(p.nf) * p.nband * p.ntiles_y * p.ntiles_x;
   const int64_t nbins = ntile_all * nsub;
-  uint32_t* counts = P->alloc<uint32_t>(size_t(nbins));
-  uint32_t* fill = P->alloc<uint32_t>(size_t(nbins));
-  int64_t* bstart = P->alloc<int64_t>(size_t(nbins));
+  Temp scratch(st);  // not needed by the cycle
+  uint32_t* counts = scratch.get<uint32_t>(size_t(nbins));
+  uint32_t* fill = scratch.get<uint32_t>(size_t(nbins));
+  int64_t* bstart = scratch.get<int64_t>(size_t(nbins));
   const int64_t ngrp = nsub < 4 ? nsub : 4;
-  uint32_t* gcount = P->alloc<uint32_t>(size_t(ntile_all * ngrp));
-  int64_t* tstart = P->alloc<int64_t>(size_t(ntile_all));
+  uint32_t* gcount = scratch.get<uint32_t>(size_t(ntile_all * ngrp));
+  int64_t* tstart = scratch.get<int64_t>(size_t(ntile_all));
   if (!counts || !fill || !bstart || !gcount || !tstart) return fail(DDF_ENOMEM, "plan allocation failed");
   HIP_TRY(hipMemsetAsync(counts, 0, size_t(nbins) * 4, st));
   HIP_TRY(hipMemsetAsync(fill, 0, size_t(nbins) * 4, st));
@@ -1768,12 +1759,6 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
   if (batched_sort_items(p, place, recs, tot, sort_items, nsort, stamp_order, st))
     return fail(DDF_EHIP, "sorting the records of the work items failed");
   HIP_TRY(hipStreamSynchronize(st));
-  // the binning buffers are not needed by the cycle
-  P->release(counts, size_t(nbins));
-  P->release(fill, size_t(nbins));
-  P->release(bstart, size_t(nbins));
-  P->release(gcount, size_t(ntile_all * ngrp));
-  P->release(tstart, size_t(ntile_all));
   *recs_out = recs;
   *items_out = d_items;
   *nrec = tot;
@@ -1982,8 +1967,9 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     const ddf_vis* v = k ? vdegrid : vgrid;
     const int64_t*& s = k ? sd : sg;
     if (s || v->nblocks == 0) continue;
+    Temp scratch(st);
     int64_t* ns = P->alloc<int64_t>(size_t(v->nblocks));
-    int64_t* tmp = P->alloc<int64_t>(size_t((v->nblocks + kScanChunk - 1) / kScanChunk));
+    int64_t* tmp = scratch.get<int64_t>(size_t((v->nblocks + kScanChunk - 1) / kScanChunk));
     if (!ns || !tmp) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
     rc = launch_bda_index(v->bda, v->nblocks, ns, tmp, st);
     if (rc) return bail(rc);
@@ -2013,30 +1999,32 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     pv->df = f2[1] - f2[0];
   }
   // placements
-  P->place_g = P->alloc<uint64_t>(size_t(vgrid->nblocks) * nfacets);
-  P->place_d = P->alloc<uint64_t>(size_t(vdegrid->nblocks) * nfacets);
-  if (!P->place_g || !P->place_d) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-  if (vgrid->nblocks && batched_place(P->pg, P->vg, false, P->place_g, st)) return bail(fail(DDF_EHIP, "plan_place failed"));
-  if (vdegrid->nblocks && batched_place(P->pd, P->vd, true, P->place_d, st)) return bail(fail(DDF_EHIP, "plan_place failed"));
+  // (of both maps, while the plan is built: ddf_plan_placements recomputes them)
+  Temp scratch_g(st), scratch_d(st);
+  uint64_t* place_g = scratch_g.get<uint64_t>(size_t(vgrid->nblocks) * nfacets);
+  uint64_t* place_d = scratch_d.get<uint64_t>(size_t(vdegrid->nblocks) * nfacets);
+  if (!place_g || !place_d) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+  if (vgrid->nblocks && batched_place(P->pg, P->vg, false, place_g, st)) return bail(fail(DDF_EHIP, "plan_place failed"));
+  if (vdegrid->nblocks && batched_place(P->pd, P->vd, true, place_d, st)) return bail(fail(DDF_EHIP, "plan_place failed"));
   // bins
   int64_t nr = 0;
-  rc = build_bins(P, P->pg, P->vg, P->place_g, chunk, &P->recs_g, &P->items_g, &nr, true, st, &P->tile_first_g, &P->tile_count_g,
+  rc = build_bins(P, P->pg, P->vg, place_g, chunk, &P->recs_g, &P->items_g, &nr, true, st, &P->tile_first_g, &P->tile_count_g,
                   nullptr, nullptr);
   if (rc) return bail(rc);
   const uint32_t ni = P->pg.nitems_b;
   P->stats[0] = nr;
   P->stats[2] = ni;
   P->bstamp_g = P->alloc<uint64_t>(size_t(nr));
-  if (!P->bstamp_g || batched_stamp_records(P->pg, P->place_g, P->recs_g, nr, P->bstamp_g, st))
+  if (!P->bstamp_g || batched_stamp_records(P->pg, place_g, P->recs_g, nr, P->bstamp_g, st))
     return bail(fail(DDF_ENOMEM, "plan allocation failed"));
   // the grid map's placements reduced to pair codes (3.5 GB -> 0.44 GB at the 81-facet chunk)
   {
     const size_t np = size_t(vgrid->nblocks) * nfacets;
     P->pcode_g = P->alloc<uint8_t>(np);
-    if (!P->pcode_g || batched_pair_codes(P->place_g, int64_t(np), P->pcode_g, st) ||
+    if (!P->pcode_g || batched_pair_codes(place_g, int64_t(np), P->pcode_g, st) ||
         hipStreamSynchronize(st) != hipSuccess)
       return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    P->release(P->place_g, np);
+    scratch_g.free();
   }
 
   {
@@ -2053,20 +2041,20 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
         return bail(fail(DDF_ENOMEM, "plan allocation failed"));
     }
   }
-  rc = build_bins(P, P->pd, P->vd, P->place_d, chunk, &P->recs_d, &P->items_d, &nr, false, st, nullptr, nullptr, &P->pa, &P->items_a);
+  rc = build_bins(P, P->pd, P->vd, place_d, chunk, &P->recs_d, &P->items_d, &nr, false, st, nullptr, nullptr, &P->pa, &P->items_a);
   if (rc) return bail(rc);
   P->stats[1] = nr;
   P->stats[3] = P->pd.nitems_b;
   P->bstamp_d = P->alloc<uint64_t>(size_t(nr));
-  if (!P->bstamp_d || batched_stamp_records(P->pd, P->place_d, P->recs_d, nr, P->bstamp_d, st))
+  if (!P->bstamp_d || batched_stamp_records(P->pd, place_d, P->recs_d, nr, P->bstamp_d, st))
     return bail(fail(DDF_ENOMEM, "plan allocation failed"));
   {
     const size_t np = size_t(vdegrid->nblocks) * nfacets;
     P->pcode_d = P->alloc<uint8_t>(np);
-    if (!P->pcode_d || batched_pair_codes(P->place_d, int64_t(np), P->pcode_d, st) ||
+    if (!P->pcode_d || batched_pair_codes(place_d, int64_t(np), P->pcode_d, st) ||
         hipStreamSynchronize(st) != hipSuccess)
       return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    P->release(P->place_d, np);
+    scratch_d.free();
   }
 
   // pass A layout
@@ -2131,9 +2119,10 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     return bail(fail(DDF_EHIP, "memset failed"));
   // visibility list of the degrid map
   if (vdegrid->nblocks) {
-    int32_t* cnt = P->alloc<int32_t>(size_t(vdegrid->nblocks));
-    int64_t* vs = P->alloc<int64_t>(size_t(vdegrid->nblocks));
-    int64_t* tmp = P->alloc<int64_t>(size_t((vdegrid->nblocks + kScanChunk - 1) / kScanChunk));
+    Temp rt(st);
+    int32_t* cnt = rt.get<int32_t>(size_t(vdegrid->nblocks));
+    int64_t* vs = rt.get<int64_t>(size_t(vdegrid->nblocks));
+    int64_t* tmp = rt.get<int64_t>(size_t((vdegrid->nblocks + kScanChunk - 1) / kScanChunk));
     if (!cnt || !vs || !tmp) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
     if (batched_vis_counts(P->vd, cnt, st)) return bail(fail(DDF_EHIP, "launch failed"));
     rc = launch_scan(cnt, vdegrid->nblocks, 0, vs, tmp, st);
@@ -2155,7 +2144,6 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     // runs of consecutive entries with one block and one Jones key: degrid pass B forms each
     // facet's Jones product once per run
     if (d.nvl >= (int64_t(1) << 32)) return bail(fail(DDF_EINVAL, "degrid visibility list too long for one plan"));
-    Temp rt(st);
     int32_t* flag = static_cast<int32_t*>(rt.get(size_t(d.nvl) * sizeof(int32_t)));
     int64_t* excl = static_cast<int64_t*>(rt.get(size_t(d.nvl) * sizeof(int64_t)));
     int64_t* ctmp = static_cast<int64_t*>(rt.get(size_t((d.nvl + kScanChunk - 1) / kScanChunk) * sizeof(int64_t)));
@@ -2291,7 +2279,7 @@ extern "C" int ddf_plan_degrid_adjoint(ddf_plan* P, const float* vis_bar, void* 
 
 extern "C" int ddf_plan_info(const ddf_plan* P, int64_t* out, int32_t n) {
   if (!P || !out) return fail(DDF_EINVAL, "null argument");
-  for (int i = 0; i < n && i < 8; ++i) out[i] = P->stats[i];
+  for (int i = 0; i < n && i < 8; ++i) out[i] = i == 5 ? int64_t(P->arena.bytes()) : P->stats[i];
   for (int i = 8; i < n && i < 11; ++i) out[i] = int64_t(P->nwg_tiles[i - 8]);
   return DDF_OK;
 }

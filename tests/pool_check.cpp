@@ -26,11 +26,13 @@ hipError_t pool_trim(size_t keep) { return note(keep == kPoolKeep ? "trim" : "ba
 int main() {
   ddf::PoolArena a, none;
   if (!a.get(100, nullptr) || !a.get(size_t(40) << 20, nullptr)) return 1;  // a slab, and a buffer of its own
+  // what is held is whole slabs and whole buffers, until the end
+  if (a.bytes() != (size_t(42) << 20) || none.bytes() != 0) return 2;
   hipSetDevice(1);
   a.close();
   none.close();
   std::string all;
   for (const std::string& s : g_log) all += s + " ";
   printf("%s-> %d\n", all.c_str(), g_dev);
-  return all == "wait0 free0 free0 sync0 trim0 " && g_dev == 1 && a.empty() ? 0 : 1;
+  return all == "wait0 free0 free0 sync0 trim0 " && g_dev == 1 && a.empty() && a.bytes() == 0 ? 0 : 1;
 }
