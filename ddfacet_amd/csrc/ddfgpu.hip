@@ -2118,10 +2118,11 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   if (hipMemsetAsync(P->M, 0, size_t(vdegrid->nblocks) * nfacets * smd.nstokes * 8, st) != hipSuccess)
     return bail(fail(DDF_EHIP, "memset failed"));
   // visibility list of the degrid map
+  Temp rt(st);
+  int64_t* vs = nullptr;
   if (vdegrid->nblocks) {
-    Temp rt(st);
     int32_t* cnt = rt.get<int32_t>(size_t(vdegrid->nblocks));
-    int64_t* vs = rt.get<int64_t>(size_t(vdegrid->nblocks));
+    vs = rt.get<int64_t>(size_t(vdegrid->nblocks));
     int64_t* tmp = rt.get<int64_t>(size_t((vdegrid->nblocks + kScanChunk - 1) / kScanChunk));
     if (!cnt || !vs || !tmp) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
     if (batched_vis_counts(P->vd, cnt, st)) return bail(fail(DDF_EHIP, "launch failed"));
@@ -2133,8 +2134,10 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
         hipMemcpyAsync(&last_cnt, cnt + vdegrid->nblocks - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
       return bail(fail(DDF_EHIP, "copy failed"));
+    P->deg.nvl = last_start + last_cnt;
+  }
+  if (P->deg.nvl > 0) {  // (blocks without visibilities leave nothing to list)
     DegridRuns& d = P->deg;
-    d.nvl = last_start + last_cnt;
     uint64_t* vrc = P->alloc<uint64_t>(size_t(d.nvl));
     uint32_t* vblk = P->alloc<uint32_t>(size_t(d.nvl));
     if (!vrc || !vblk) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
