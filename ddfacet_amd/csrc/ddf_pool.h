@@ -50,6 +50,17 @@ class PoolArena {
     left_ = bytes_ = 0;
   }
   size_t bytes() const { return bytes_; }  // of device memory held
+  // takes over the buffers of another arena of the same device
+  void take(PoolArena& o) {
+    if (empty()) dev_ = o.dev_;
+    own_.insert(own_.end(), o.own_.begin(), o.own_.end());
+    own_.insert(own_.end(), o.slabs_.begin(), o.slabs_.end());
+    bytes_ += o.bytes_;
+    o.own_.clear();
+    o.slabs_.clear();
+    o.cur_ = nullptr;
+    o.left_ = o.bytes_ = 0;
+  }
   bool empty() const { return own_.empty() && slabs_.empty(); }
   // Gives everything back at the end of an object whose work may still run on any stream: waits for the device of
   // the buffers, whichever one is current, and hands what the pool does not keep to the device before it returns.

@@ -1767,6 +1767,51 @@ int build_bins(ddf_plan* P, BatchParams& p, const VisP& v, const uint64_t* place
 
 }  // namespace
 
+namespace {
+
+// The run list of the grid map, for grid_pass_a_runs.  It is left out where a plan does not take it or where its
+// 8 bytes a visibility cannot be had: grid_pass_a grids the map then.
+int build_runs(ddf_plan* P, const ddf_vis* v, int group, hipStream_t st) {
+  RunList rl = {};
+  if (!batched_runs_layout(P->pg, P->vg, group, &rl)) return DDF_OK;
+  const int64_t nb = v->nblocks;
+  Temp rt(st), list(st);
+  auto leave = [] {
+    (void)hipGetLastError();
+    return int(DDF_OK);
+  };
+  int32_t* cnt = rt.get<int32_t>(size_t(nb));
+  int64_t* tmp = rt.get<int64_t>(size_t((nb + kScanChunk - 1) / kScanChunk));
+  int64_t* start = list.get<int64_t>(size_t(nb) + 1);
+  if (!cnt || !tmp || !start) return leave();
+  if (batched_vis_counts(P->vg, cnt, st)) return fail(DDF_EHIP, "launch failed");
+  int rc = launch_scan(cnt, nb, 0, start, tmp, st);
+  if (rc) return rc;
+  int64_t last_start = 0;
+  int32_t last_cnt = 0;
+  if (hipMemcpyAsync(&last_start, start + nb - 1, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
+      hipMemcpyAsync(&last_cnt, cnt + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+      hipStreamSynchronize(st) != hipSuccess)
+    return fail(DDF_EHIP, "copy failed");
+  const int64_t total = last_start + last_cnt;
+  batched_run_split(total, &rl);
+  uint64_t* entry = list.get<uint64_t>(size_t(total));
+  uint32_t* item = list.get<uint32_t>(size_t(rl.nitems) + 1);
+  if (!entry || !item) return leave();
+  rl.start = start;
+  if (hipMemcpyAsync(start + nb, &total, 8, hipMemcpyHostToDevice, st) != hipSuccess ||
+      hipStreamSynchronize(st) != hipSuccess || batched_run_entries(P->pg, P->vg, start, entry, st) ||
+      batched_run_items(P->vg, rl, item, st))
+    return fail(DDF_EHIP, "launch failed");
+  rl.item = item;
+  rl.entry = entry;
+  P->runs = rl;
+  P->arena.take(list.arena);
+  return DDF_OK;
+}
+
+}  // namespace
+
 extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, const ddf_vis* vdegrid,
                                const ddf_facet* facets, void* const* models, int32_t nfacets,
                                const ddf_plan_opts* opts, ddf_plan** out, void* stream) {
@@ -2035,10 +2080,13 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     const size_t n = size_t(ni) * size_t(npg) * 2 * size_t(W) * size_t(W);
     if (ni) {
       P->slots_g = P->alloc<float>(n);
-      if (!P->slots_g) (void)hipGetLastError();
-      P->live_g = P->alloc<uint32_t>(1 + size_t(nfacets) * g->nband * P->pg.ntiles_y * P->pg.ntiles_x);
-      if (!P->live_g || batched_live_tiles(P->pg, P->tile_count_g, P->live_g, st))
-        return bail(fail(DDF_ENOMEM, "plan allocation failed"));
+      if (P->slots_g) P->live_g = P->alloc<uint32_t>(1 + size_t(nfacets) * g->nband * P->pg.ntiles_y * P->pg.ntiles_x);
+      if (!P->live_g) {
+        P->slots_g = nullptr;
+        (void)hipGetLastError();
+      } else if (batched_live_tiles(P->pg, P->tile_count_g, P->live_g, st)) {
+        return bail(fail(DDF_EHIP, "launch failed"));
+      }
     }
   }
   rc = build_bins(P, P->pd, P->vd, place_d, chunk, &P->recs_d, &P->items_d, &nr, false, st, nullptr, nullptr, &P->pa, &P->items_a);
@@ -2076,36 +2124,6 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
                    (size_t(nfacets) * per_f + size_t(G) * (2 * size_t(vgrid->nchan) + 1)) * 8 + stage_bytes <= 80 * 1024;
   if (size_t(nfacets) * per_f * 8 + stage_bytes > 80 * 1024)
     return bail(fail(DDF_EINVAL, "facets x bands too large for one plan"));
-  // the run list of the grid map
-  if (batched_runs_layout(P->pg, P->vg, o.group, &P->runs)) {
-    const int64_t nb = vgrid->nblocks;
-    Temp rt(st);
-    int32_t* cnt = static_cast<int32_t*>(rt.get(size_t(nb) * 4));
-    int64_t* tmp = static_cast<int64_t*>(rt.get(size_t((nb + kScanChunk - 1) / kScanChunk) * 8));
-    int64_t* start = P->alloc<int64_t>(size_t(nb) + 1);
-    if (!cnt || !tmp || !start) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    if (batched_vis_counts(P->vg, cnt, st)) return bail(fail(DDF_EHIP, "launch failed"));
-    rc = launch_scan(cnt, nb, 0, start, tmp, st);
-    if (rc) return bail(rc);
-    int64_t last_start = 0;
-    int32_t last_cnt = 0;
-    if (hipMemcpyAsync(&last_start, start + nb - 1, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(&last_cnt, cnt + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-      return bail(fail(DDF_EHIP, "copy failed"));
-    const int64_t total = last_start + last_cnt;
-    if (total >= (int64_t(1) << 36)) return bail(fail(DDF_EINVAL, "visibility list too long for one plan"));
-    uint64_t* entry = P->alloc<uint64_t>(size_t(total));
-    if (!entry || hipMemcpyAsync(start + nb, &total, 8, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess || batched_run_entries(P->pg, P->vg, start, entry, st))
-      return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    P->runs.start = start;
-    batched_run_split(total, &P->runs);
-    uint32_t* item = P->alloc<uint32_t>(size_t(P->runs.nitems) + 1);
-    if (!item || batched_run_items(P->vg, P->runs, item, st)) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
-    P->runs.item = item;
-    P->runs.entry = entry;
-  }
   // LDS tiles
   const int W = tile + 2 * halo;
   const int npg = smg.nstokes < g->npol ? smg.nstokes : g->npol;
@@ -2215,6 +2233,9 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
   } else if (batched_tile_wgs(P->pg, P->pd, P->nwg_tiles)) {
     return bail(fail(DDF_EHIP, "occupancy query failed"));
   }
+  // (last: everything else comes before its memory)
+  rc = build_runs(P, vgrid, o.group, st);
+  if (rc) return bail(rc);
   if (hipStreamSynchronize(st) != hipSuccess) return bail(fail(DDF_EHIP, "plan build failed"));
   *out = P;
   return DDF_OK;

@@ -24,8 +24,11 @@ hipError_t pool_trim(size_t keep) { return note(keep == kPoolKeep ? "trim" : "ba
 }  // namespace ddf
 
 int main() {
-  ddf::PoolArena a, none;
-  if (!a.get(100, nullptr) || !a.get(size_t(40) << 20, nullptr)) return 1;  // a slab, and a buffer of its own
+  ddf::PoolArena a, none, list;
+  // a slab, and a buffer of its own, made as an optional list's that the owner then takes over
+  if (!list.get(100, nullptr) || !list.get(size_t(40) << 20, nullptr)) return 1;
+  a.take(list);
+  if (!list.empty() || list.bytes() != 0) return 3;
   // what is held is whole slabs and whole buffers, until the end
   if (a.bytes() != (size_t(42) << 20) || none.bytes() != 0) return 2;
   hipSetDevice(1);
