@@ -1186,7 +1186,11 @@ __global__ __launch_bounds__(64 * kRunWaves) void grid_pass_a_runs(BatchParams p
       S.u2[lane] = u2;
       // run starts, valid entries, and each channel's weight over its run: the entries of a run are rows
       // of `width` channels, so the first `width` of them hold each channel once
-      const uint64_t runs = __ballot(lane < nent && ((rc >> 63) != 0 || lane == 0)), valids = __ballot(valid);
+      // (an entry also starts one where its Jones are others than its predecessor's by the maps as they are now:
+      // the list's runs are those of the maps that the plan was built with)
+      uint32_t other = (uint32_t(__shfl_up(int(k0), 1, 64)) ^ k0) | (uint32_t(__shfl_up(int(k1), 1, 64)) ^ k1);
+      if (!J32) other |= (uint32_t(__shfl_up(int(bm0), 1, 64)) ^ bm0) | (uint32_t(__shfl_up(int(bm1), 1, 64)) ^ bm1);
+      const uint64_t runs = __ballot(lane < nent && (lane == 0 || (rc >> 63) != 0 || other != 0)), valids = __ballot(valid);
       {
         const uint64_t below = runs & ((2ull << lane) - 1), above = runs & ~((2ull << lane) - 1);
         const int rs = below ? 63 - __builtin_clzll(below) : 0, re = above ? __builtin_ctzll(above) : nent;
