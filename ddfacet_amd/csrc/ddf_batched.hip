@@ -617,9 +617,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
     }
   };
 
-  for (bool first = true;; first = false) {
+  while (true) {
     if (threadIdx.x == 0) {
-      s_item = first ? blockIdx.x : gridDim.x + atomicAdd(queue, 1u);
+      s_item = atomicAdd(queue, 1u);
       s_next = 0;
     }
     __syncthreads();
