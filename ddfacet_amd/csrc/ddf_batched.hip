@@ -2604,8 +2604,8 @@ __global__ __launch_bounds__(256) void degrid_adj_b(BatchParams p, const VisP v,
   const int lf = threadIdx.x - slot * G;
   const bool active = slot < slots;
   __shared__ uint32_t s_item;
-  for (bool first = true;; first = false) {
-    if (threadIdx.x == 0) s_item = first ? blockIdx.x : gridDim.x + atomicAdd(queue, 1u);
+  while (true) {
+    if (threadIdx.x == 0) s_item = atomicAdd(queue, 1u);
     __syncthreads();
     const uint32_t item = s_item;
     if (item >= p.nitems_a) break;
