@@ -298,13 +298,21 @@ struct DegridRuns {
   int64_t nvl = 0, nruns = 0, nquads = 0;
 };
 // Whether degrid pass B can take runs as quads: the mixed precision, and no Jones or the complex64 tables
-// (the general Jones need the registers that its four wavefronts a SIMD share).  A plan does so where a
-// quad holds at least kQuadFill visibilities on average (81 facets with Jones, 3.1 a quad: 4.56 ms, 5.3 by
-// visibility; 121 facets without, 2.5 a quad: 226 us, 359; one a quad, 1.1 M of them, 25 facets: 328 us,
-// 283), or where its tiles of 64 quads are too few for the card's 256 compute units, where tiles of
-// 256 visibilities would be fewer still (1260 visibilities, one a quad: 9.3 us, 15.9).
+// (the general Jones need the registers that its four wavefronts a SIMD share).
 bool batched_quads_take(const BatchParams& p);
-constexpr int64_t kQuadFill = 2, kQuadsFew = 64 * 256;
+// Whether it should, for a list of nvl visibilities in nruns runs, nquads quads and nf facets.  A quad costs some
+// 50 units for its tile and 1.5 a facet, a visibility by itself 10 and 1 a facet, so quads have to be filled
+// (4 visibilities or nearly so with few facets, 2.5 with many), and with Jones Y of a (run, facet) costs a unit more
+// in quads.  A list of at most 64 * 256 quads goes in quads whatever their fill: its tiles of 64 quads are too few for
+// the card's 256 compute units, and tiles of 256 visibilities would be fewer still.  4.8 M visibilities, quads and
+// by visibility, ms: 1 facet 2 a quad 0.28, 0.17; 9 facets 2.5 a quad 0.30, 0.24, 4 a quad 0.22, 0.26; 81 facets 2.5 a quad
+// 1.08, 1.14, 4 a quad 0.69, 0.91; with Jones 1 facet 2.9 a quad 0.35, 0.20; 25 facets 2.5 a quad 0.94, 0.77; 81
+// facets 2.9 a quad 1.58, 1.70, and with 19.4 M visibilities, 3.1 a quad, 4.56, 5.3.  1260 visibilities, one a quad, 9 facets:
+// 10.7 us, 16.  (Over 106 such cases the rule takes the slower one by 0.2 % on average and 6 % at most.)
+constexpr int64_t kQuadsFew = 64 * 256;
+inline bool quads_pay(int64_t nvl, int64_t nruns, int64_t nquads, int nf, bool jones) {
+  return nquads <= kQuadsFew || 2 * nvl * (10 + nf) > nquads * (100 + 3 * int64_t(nf)) + (jones ? 2 * nruns * nf : 0);
+}
 int batched_degrid_b(const BatchParams& p, const VisP& v, const float2* M, const DegridRuns& d, hipStream_t st);
 int batched_fold(const int32_t* flag, const int64_t* excl, int64_t nvl, int nf, uint8_t* fold, hipStream_t st);
 int batched_quad_counts(const DegridRuns& d, int32_t* cnt, hipStream_t st);

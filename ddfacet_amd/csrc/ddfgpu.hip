@@ -2191,14 +2191,16 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     d.run_first = run_first;
     if (batched_run_ids(P->pd, P->vd, vrc, vblk, d.nvl, flag, excl, nullptr, run_first, 1, st))
       return bail(fail(DDF_EHIP, "launch failed"));
-    if (batched_quads_take(P->pd) && (d.nruns <= d.nvl / kQuadFill || d.nruns <= kQuadsFew)) {
+    const bool jones = P->pd.jmode != 0;
+    // (no fewer quads than runs, nor than a fourth of the visibilities)
+    if (batched_quads_take(P->pd) && quads_pay(d.nvl, d.nruns, std::max(d.nruns, (d.nvl + 3) / 4), nfacets, jones)) {
       int32_t* cnt4 = static_cast<int32_t*>(rt.get(size_t(d.nruns) * sizeof(int32_t)));
       int64_t* first4 = static_cast<int64_t*>(rt.get(size_t(d.nruns) * sizeof(int64_t)));
       if (!cnt4 || !first4) return bail(fail(DDF_ENOMEM, "plan allocation failed"));
       if (batched_quad_counts(d, cnt4, st)) return bail(fail(DDF_EHIP, "launch failed"));
       rc = scan_total(cnt4, d.nruns, first4, &d.nquads);
       if (rc) return bail(rc);
-      if (d.nquads * kQuadFill <= d.nvl || d.nquads <= kQuadsFew) {
+      if (quads_pay(d.nvl, d.nruns, d.nquads, nfacets, jones)) {
         uint32_t* run_quad = P->alloc<uint32_t>(size_t(d.nruns));
         uint32_t* quad_run = P->alloc<uint32_t>(size_t((d.nquads + 63) / 64));
         uint8_t* fold = P->alloc<uint8_t>(size_t((d.nvl + 255) / 256));
