@@ -629,19 +629,25 @@ int fft_planes(const FftDims& d, float2* planes, int64_t nplanes, int inverse, d
   while (lc > 2 && fft_lds_bytes(n, 1 << lc) > 80 * 1024) --lc;
   const int strips = (n + (1 << lc) - 1) >> lc;
   int rows = int(32 * 1024 / (size_t(n) * 8));
-  const int64_t nrow = nplanes * n;
-  rows = int(std::max<int64_t>(1, std::min<int64_t>({16, rows, nrow / 512})));
-  if (nrow >= (int64_t(1) << 31)) return ifail(DDF_EINVAL, "too many planes for one FFT call");
-  const dim3 g(unsigned(nplanes * strips)), b(512);
+  rows = int(std::max<int64_t>(1, std::min<int64_t>({16, rows, nplanes * n / 512})));
+  const dim3 b(512);
   const size_t lds = fft_lds_bytes(n, 1 << lc);
-  if (lc == 4) hipLaunchKernelGGL((fft_columns<4>), g, b, lds, st, d, planes, fp, strips);
-  else if (lc == 3) hipLaunchKernelGGL((fft_columns<3>), g, b, lds, st, d, planes, fp, strips);
-  else hipLaunchKernelGGL((fft_columns<2>), g, b, lds, st, d, planes, fp, strips);
-  HIP_OK(hipGetLastError());
-  fp.scale = float(norm);
-  hipLaunchKernelGGL(fft_rows, dim3(unsigned((nrow + rows - 1) / rows)), dim3(256), fft_lds_bytes(n, rows), st, d, planes, fp,
-                     rows, nrow);
-  HIP_OK(hipGetLastError());
+  // a launch takes fewer than 2^32 threads: 2^22 strips of 512 at most, and no more rows than fit as well
+  const int64_t most = (int64_t(1) << 22) / strips;
+  for (int64_t p0 = 0; p0 < nplanes; p0 += most) {
+    const int64_t np = std::min(most, nplanes - p0), nrow = np * n;
+    float2* a = planes + p0 * n * n;
+    const dim3 g(unsigned(np * strips));
+    fp.scale = 1.f;
+    if (lc == 4) hipLaunchKernelGGL((fft_columns<4>), g, b, lds, st, d, a, fp, strips);
+    else if (lc == 3) hipLaunchKernelGGL((fft_columns<3>), g, b, lds, st, d, a, fp, strips);
+    else hipLaunchKernelGGL((fft_columns<2>), g, b, lds, st, d, a, fp, strips);
+    HIP_OK(hipGetLastError());
+    fp.scale = float(norm);
+    hipLaunchKernelGGL(fft_rows, dim3(unsigned((nrow + rows - 1) / rows)), dim3(256), fft_lds_bytes(n, rows), st, d, a, fp,
+                       rows, nrow);
+    HIP_OK(hipGetLastError());
+  }
   return DDF_OK;
 }
 
