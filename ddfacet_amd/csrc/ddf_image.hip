@@ -785,6 +785,10 @@ extern "C" int ddf_stitch(const ddf_image_facet* facets, int32_t nf, int32_t npi
   for (int i = 0; i < nf; ++i)
     if (!facets[i].dirty || !facets[i].inv_sphe || !facets[i].sumwt) return ifail(DDF_EINVAL, "facet buffer is null");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // a graph would keep the address of this call's list of facets, and read it at every replay
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capture) != hipSuccess) (void)hipGetLastError();
+  if (capture != hipStreamCaptureStatusNone) return ifail(DDF_EHIP, "ddf_stitch cannot be captured into a graph");
   std::vector<void*> tmp;
   TmpFree guard{tmp, st};
   ImgFacet* d = nullptr;
