@@ -121,9 +121,15 @@ int get_plan(int n, int64_t nplanes, int inverse, FFTPlan** out) {
   return DDF_OK;
 }
 
+// LDS of a pass: `count` transforms of n points, the twiddles and the places of the frequencies.
+constexpr size_t fft_lds_bytes(int n, int count) { return size_t(n) * (count + 1) * 8 + size_t(n) * 2; }
+constexpr size_t kFftLds = 80 * 1024;  // for two workgroups a CU
+
 // Factors and device tables of a length (made once per length and device, 12 n bytes); false where the
 // passes do not take it: a prime factor above 13, or a length whose strip of four columns no longer
-// leaves room for two workgroups on a CU (above 2048; a strip of two is read in 16-byte pieces).
+// leaves room for two workgroups on a CU (above 1950; a strip of two is read in 16-byte pieces).  24 planes,
+// passes and rocFFT: 1944 points 1.47 ms, 1.71; with one workgroup a CU 1960 points 1.98, 1.86 and 2048 points
+// 2.20, 1.85.
 std::map<std::pair<int, int>, FftDims> g_fft_dims;  // (n, device)
 
 int fft_dims(int n, FftDims* out, bool* ok) {
@@ -144,7 +150,7 @@ int fft_dims(int n, FftDims* out, bool* ok) {
       d.rcp_b[s] = nb > 1 ? uint32_t(((uint64_t(1) << 32) + nb - 1) / nb) : 0;
     }
   }
-  if (left != 1 || n > 2048) return DDF_OK;
+  if (left != 1 || fft_lds_bytes(n, 4) > kFftLds) return DDF_OK;
   d.rcp_n = n > 1 ? uint32_t(((uint64_t(1) << 32) + n - 1) / n) : 0;
   int dev = 0;
   HIP_OK(hipGetDevice(&dev));
@@ -486,7 +492,6 @@ __device__ __forceinline__ FftLds fft_lds_setup(float2* lds, const FftDims& d, i
   }
   return l;
 }
-inline size_t fft_lds_bytes(int n, int count) { return size_t(n) * (count + 1) * 8 + size_t(n) * 2; }
 
 template <int LOGC>
 __global__ __launch_bounds__(512) void fft_columns(FftDims d, float2* planes, FftPass fp, int strips) {
@@ -619,14 +624,14 @@ int upload_facets(const ddf_image_facet* facets, int nf, int n, int m, hipStream
 }
 
 // The centred transform of `nplanes` planes by the passes.  Columns of a strip: the most of 16, 8 and 4
-// that leave two workgroups a CU (80 KB of LDS each); rows of a workgroup: about 32 KB, at most 16.
-// Fewer rows where the launch would not give every CU two workgroups.
+// that leave two workgroups a CU (80 KB of LDS each: 16 to 593 points, 8 to 1107, 4 to 1950); rows of a
+// workgroup: about 32 KB, at most 16.  Fewer rows where the launch would not give every CU two workgroups.
 int fft_planes(const FftDims& d, float2* planes, int64_t nplanes, int inverse, double scale, hipStream_t st) {
   const int n = d.n;
   const double norm = inverse ? scale : scale / (double(n) * double(n));
   FftPass fp{n / 2, (n + 1) / 2, inverse != 0, 1.f};
   int lc = 4;
-  while (lc > 2 && fft_lds_bytes(n, 1 << lc) > 80 * 1024) --lc;
+  while (fft_lds_bytes(n, 1 << lc) > kFftLds) --lc;  // (fft_dims: a strip of four fits)
   const int strips = (n + (1 << lc) - 1) >> lc;
   int rows = int(32 * 1024 / (size_t(n) * 8));
   rows = int(std::max<int64_t>(1, std::min<int64_t>({16, rows, nplanes * n / 512})));
