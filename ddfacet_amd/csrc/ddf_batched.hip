@@ -2954,13 +2954,26 @@ static DegridPassA degrid_pass_a_for(int prec, bool one) {
 
 // Persistent grid sizes of the tile passes (grid B, degrid A, adjoint of degrid A), computed once
 // per plan so that the launches make no device queries (they may run under stream capture).
-int batched_tile_wgs(const BatchParams& pg, const BatchParams& pd, unsigned out[3]) {
+int batched_tile_wgs(const BatchParams& pg, BatchParams& pd, unsigned out[3]) {
   const int Wg = pg.tile + 2 * pg.halo, Wd = pd.tile + 2 * pd.halo;
   const int npg = pg.nstokes < pg.npol ? pg.nstokes : pg.npol;
   const int npd = pd.nstokes < pd.npol ? pd.nstokes : pd.npol;
   out[0] = persistent_wgs(grid_pass_b_for<false, false>(npg, pg.halo), grid_pass_b_lds(npg, Wg, false), 0, 64);
   const size_t lds_d = size_t(pd.nstokes) * Wd * Wd * 2 * sizeof(float);
-  out[1] = persistent_wgs(degrid_pass_a_for(pd.prec, pd.nstokes == 1), lds_d, 0, pd.tile_threads);
+  // Degrid pass A takes four wavefronts an item, or one where only so every pack has a workgroup of its own: each
+  // further pack is an atomic on the queue's counter (12 ns in turn), and four wavefronts a workgroup leave 2048
+  // workgroups, one 8192.  9 facets: 5100 items of 40 records 22 us with one, 75 with four; 6700 of 241 75 and
+  // 95, 7200 of 414 134 and 113; 8900 of 46, which have to queue either way, 124 and 116.  One facet, 430 items of 26:
+  // 11.8 and 10.2; 81 facets, 34 000 items of 184: 586 and 428.
+  const DegridPassA ka = degrid_pass_a_for(pd.prec, pd.nstokes == 1);
+  out[1] = persistent_wgs(ka, lds_d, 0, 256);
+  if (pd.npacks > out[1] && pd.tile_records < int64_t(pd.nitems_b) * 320) {
+    const unsigned n = persistent_wgs(ka, lds_d, 0, 64);
+    if (pd.npacks <= n) {
+      out[1] = n;
+      pd.tile_threads = 64;
+    }
+  }
   out[2] = persistent_wgs(grid_pass_b_adjoint_for(npd, pd.halo, Wd, pd.prec),
                           grid_pass_b_lds(npd, Wd, adjoint_wide(npd, Wd, pd.prec)), 0, 64);
   return hipGetLastError() == hipSuccess ? DDF_OK : DDF_EHIP;

@@ -220,7 +220,8 @@ struct BatchParams {
   // range x is packs [pack_range[x], pack_range[x + 1])
   const uint32_t* pack_range;
   int nranges;
-  int tile_threads;  // workgroup of degrid pass A
+  int64_t tile_records;  // records of the work items
+  int tile_threads;      // workgroup of degrid pass A (batched_tile_wgs)
   // blocks of the pass's BDA map: the per-(block, facet) values between the passes are stored
   // facet-major, [facet][block][nstokes]
   int64_t nblk;
@@ -328,7 +329,7 @@ int batched_degrid_b_adjoint(const BatchParams& p, const VisP& v, const uint8_t*
 int batched_degrid_a_adjoint(const BatchParams& p, const uint64_t* place, const float2* Mbar, const BinItem* items,
                              const uint32_t* recs, uint32_t* queue, unsigned nwg, hipStream_t st);
 
-int batched_tile_wgs(const BatchParams& pg, const BatchParams& pd, unsigned out[3]);
+int batched_tile_wgs(const BatchParams& pg, BatchParams& pd, unsigned out[3]);
 // stamp records (tile offset | support << 16 | CF offset << 32) of the binned records
 int batched_stamp_records(const BatchParams& p, const uint64_t* place, const uint32_t* recs, int64_t n,
                           uint64_t* bstamp, hipStream_t st);

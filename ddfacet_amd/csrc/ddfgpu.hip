@@ -1677,8 +1677,7 @@ int upload_items(ddf_plan* P, BatchParams& p, const TileItems& L, BinItem** item
   p.npacks = uint32_t(L.packs.size()) - 1;
   p.nranges = L.nranges;
   p.nitems_b = uint32_t(L.items.size());
-  // degrid pass A: a workgroup of one wavefront where an item has few records for four
-  p.tile_threads = L.records < int64_t(L.items.size()) * 192 ? 64 : 256;
+  p.tile_records = L.records;
   *items_out = d_items;
   return DDF_OK;
 }
@@ -2230,6 +2229,7 @@ extern "C" int ddf_plan_create(const ddf_grid_desc* g, const ddf_vis* vgrid, con
     return bail(fail(DDF_EHIP, "device query failed"));
   P->nwg = unsigned(o.workgroups > 0 ? o.workgroups : prop.multiProcessorCount * 4);
   P->nwg_runs = unsigned(o.workgroups > 0 ? o.workgroups : prop.multiProcessorCount);
+  P->pd.tile_threads = 256;
   if (o.workgroups > 0) {
     for (unsigned& x : P->nwg_tiles) x = unsigned(o.workgroups);
   } else if (batched_tile_wgs(P->pg, P->pd, P->nwg_tiles)) {
