@@ -162,6 +162,8 @@ struct KParams {
   int nstokes;
   double sm[4][4][2];
   int chan_lds;   // per-channel Jones sums accumulated in LDS (else straight to global)
+  int64_t large;       // visibilities of a large block: the first large_wgs workgroups take those
+  unsigned large_wgs;
 };
 
 __device__ __forceinline__ cd smc(const KParams& p, int r, int c) { return cd{p.sm[r][c][0], p.sm[r][c][1]}; }
@@ -170,9 +172,11 @@ __device__ __forceinline__ cd smc(const KParams& p, int r, int c) { return cd{p.
 // A wavefront takes 64 / GS consecutive blocks, GS = 1 << LG lanes each: the lanes of a group walk their
 // block's rows and visibilities (channel fastest) and add up their partial sums by a butterfly within
 // the group; then the whole wavefront takes the stamps of its blocks one after the other, lanes over
-// cells, the next stamp's CF values in flight with the current one.  GS is the power of two at or
-// below the map's mean visibilities per block (plain_group): with a wavefront per block, a block of one
-// visibility left 63 lanes idle through the phase, the Jones products and the placement.
+// cells, the next stamp's CF values in flight with the current one.  GS follows the map's mean visibilities
+// per block (plain_group): with a wavefront per block, a block of one visibility left 63 lanes idle through
+// the phase, the Jones products and the placement.  An averaging map has blocks of hundreds of visibilities
+// beside its single ones: with 1 or 8 lanes a block these are left to the first workgroups of the launch,
+// which look through the map and give each a wavefront.
 template <int LG>
 __device__ __forceinline__ double group_sum(double v) {
 #pragma unroll
@@ -192,6 +196,31 @@ __device__ __forceinline__ int64_t read_lane(int64_t x, int j) {
 }
 __device__ __forceinline__ double read_lane(double x, int j) {
   return __builtin_bit_cast(double, read_lane(__builtin_bit_cast(int64_t, x), j));
+}
+
+// The wavefronts of a part of the launch, and this one's place among them.
+struct Part {
+  int64_t wave, nwaves;
+};
+template <int LG>
+__device__ __forceinline__ Part plain_part(const KParams& p, bool large) {
+  const unsigned wgs = LG == 6 ? gridDim.x : large ? p.large_wgs : gridDim.x - p.large_wgs;
+  const unsigned wg = LG == 6 || large ? blockIdx.x : blockIdx.x - p.large_wgs;
+  return Part{(int64_t(wg) * blockDim.x + threadIdx.x) >> 6, (int64_t(wgs) * blockDim.x) >> 6};
+}
+// The kernel's parameters, read again: with one set of loads for both parts of a launch the compiler holds them over the
+// branch and spills for it.
+__device__ __forceinline__ const KParams& own_params() {
+  auto q = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));
+  return *(const KParams*)q;
+}
+// The large ones of the blocks b0, b0 + nwaves, ... (neighbours, often of one baseline and large together, go to
+// different wavefronts so).
+__device__ __forceinline__ uint64_t large_blocks(const KParams& p, int64_t b0, int64_t nwaves) {
+  const int64_t b = b0 + (threadIdx.x & 63) * nwaves;
+  const BlockRec br = read_block(p.v, b < p.v.nblocks ? b : 0);
+  return __ballot(b < p.v.nblocks && int64_t(br.nr) * (br.ch1 - br.ch0) > p.large);
 }
 
 // Block means over the unflagged (row, channel) visibilities (gridder.h:272-289).
@@ -230,32 +259,22 @@ __device__ inline Means block_means(const KParams& p, const BlockRec& br, int64_
 // of one cell, so that a line of the grid is touched once a stamp and not once for either part.
 // 561 600 blocks of one visibility, 7 x 7 stamps: 1.60 ms with a wavefront per block, 0.51 here
 // (0.19 of it without the atomics; 0.64 with 8 lanes per block).
-template <int READ, int JMODE, typename GT, int LG>
-__global__ __launch_bounds__(256) void grid_plain(KParams p) {
-  extern __shared__ double lds[];
+template <int READ, int JMODE, typename GT, int LG, bool LARGE>
+__device__ __forceinline__ void grid_part(const KParams& p, const Part& part, double* s_sumwt, double* s_sj, double* s_sjc) {
   constexpr int GS = 1 << LG, NB = kWave / GS;
-  const int nbp = p.nband * p.npol;
-  double* s_sumwt = lds;                       // [nband*npol]
-  double* s_sj = lds + nbp;                    // [2*nband]
-  double* s_sjc = lds + nbp + 2 * p.nband;     // [2*nchan] when chan_lds
-  const int nacc = nbp + 2 * p.nband + (p.chan_lds ? 2 * p.v.nchan : 0);
-  for (int i = threadIdx.x; i < nacc; i += blockDim.x) lds[i] = 0.;
-  __syncthreads();
-
   const int lane = threadIdx.x & 63, sub = lane & (GS - 1), grp = lane >> LG;
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-  const int64_t nwaves = (int64_t(gridDim.x) * blockDim.x) >> 6;
+  const int64_t wave = part.wave, nwaves = part.nwaves;
   const VisP& v = p.v;
   DDF_GLOBAL GT* grid = gptr_w(reinterpret_cast<GT*>(p.grid));
   const int npg = p.nstokes < p.npol ? p.nstokes : p.npol;
   double* sjc = p.chan_lds ? s_sjc : p.jp.sum_jones_chan;
 
-  for (int64_t b0 = wave * NB; b0 < v.nblocks; b0 += nwaves * NB) {
-    const int64_t b = b0 + grp;
+  auto block = [&](int64_t b) {  // of this group of lanes
     const bool mine = b < v.nblocks && !(v.sparse && !v.sparse[b]);
     const BlockRec br = read_block(v, mine ? b : 0);
     const int nch = br.ch1 - br.ch0;
-    const int64_t nvis = mine ? int64_t(br.nr) * nch : 0;
+    const int64_t size = int64_t(br.nr) * nch;
+    const int64_t nvis = mine && (LG == 6 || size <= p.large) ? size : 0;
     const int64_t mid = nvis > 0 ? int64_t(br.rows[br.nr / 2]) : -1;
     const bool mid_ok = mid >= 0 && mid < v.nrow;
     const double dec = mid_ok ? decorr_factor(p.dp, v.uvw, p.tscale0, mid) : 1.;
@@ -425,7 +444,31 @@ __global__ __launch_bounds__(256) void grid_plain(KParams p) {
         }
       }
     }
+  };
+  for (int64_t b0 = wave * NB; b0 < v.nblocks; b0 += nwaves * (LARGE ? kWave : NB)) {
+    if (LARGE) {
+      for (uint64_t take = large_blocks(p, b0, nwaves); take; take &= take - 1) block(b0 + __builtin_ctzll(take) * nwaves);
+    } else {
+      block(b0 + grp);
+    }
   }
+}
+
+template <int READ, int JMODE, typename GT, int LG>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void grid_plain(KParams p) {
+  extern __shared__ double lds[];
+  const int nbp = p.nband * p.npol;
+  double* s_sumwt = lds;                       // [nband*npol]
+  double* s_sj = lds + nbp;                    // [2*nband]
+  double* s_sjc = lds + nbp + 2 * p.nband;     // [2*nchan] when chan_lds
+  const int nacc = nbp + 2 * p.nband + (p.chan_lds ? 2 * p.v.nchan : 0);
+  for (int i = threadIdx.x; i < nacc; i += blockDim.x) lds[i] = 0.;
+  __syncthreads();
+  if (LG < 6 && blockIdx.x < p.large_wgs) {
+    const KParams& q = own_params();
+    grid_part<READ, JMODE, GT, 6, true>(q, plain_part<LG>(q, true), s_sumwt, s_sj, s_sjc);
+  } else
+    grid_part<READ, JMODE, GT, LG, false>(p, plain_part<LG>(p, false), s_sumwt, s_sj, s_sjc);
   __syncthreads();
   for (int i = threadIdx.x; i < nbp; i += blockDim.x)
     if (s_sumwt[i] != 0.) atomicAdd(&p.sumwt[i], s_sumwt[i]);
@@ -439,24 +482,22 @@ __global__ __launch_bounds__(256) void grid_plain(KParams p) {
 }
 
 // ---- degridding kernel ---------------------------------------------------------------------
-// Stamps of up to 256 cells are gathered with the next block's values in flight.  2.25 M visibilities in
-// 160 000 blocks with DD Jones: 1.72 ms with a wavefront per block, DE0.51 here
-// (0.19 of it without the atomics; 0.64 with 8 lanes per block).
-// (Three wavefronts per SIMD: the FP64 Jones products held 253 registers, 375 us against 399.)
-template <int NCORR, int JMODE, int LG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void degrid_plain(KParams p) {
+// Bound by the FP64 phase and Jones products of every visibility.  Stamps of up to 256 cells are gathered with the
+// next block's values in flight.  2.25 M visibilities in 509 000 blocks with DD Jones: 1.72 ms with a wavefront
+// per block, 0.36 with 8 lanes and no large blocks apart, 0.27 here.
+// (Three wavefronts per SIMD with Jones: the FP64 products held 253 registers, 375 us against 399 with 8 lanes.)
+template <int NCORR, int JMODE, int LG, bool LARGE>
+__device__ __forceinline__ void degrid_part(const KParams& p, const Part& part) {
   constexpr int GS = 1 << LG, NB = kWave / GS;
   const int lane = threadIdx.x & 63, sub = lane & (GS - 1), grp = lane >> LG;
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
-  const int64_t nwaves = (int64_t(gridDim.x) * blockDim.x) >> 6;
+  const int64_t wave = part.wave, nwaves = part.nwaves;
   const VisP& v = p.v;
   const DDF_GLOBAL float2* grid = gptr(reinterpret_cast<const float2*>(p.grid));
 
-  for (int64_t b0 = wave * NB; b0 < v.nblocks; b0 += nwaves * NB) {
-    const int64_t b = b0 + grp;
+  auto block = [&](int64_t b) {  // of this group of lanes
     const BlockRec br = read_block(v, b < v.nblocks ? b : 0);
     const int nch = br.ch1 - br.ch0;
-    const bool some = b < v.nblocks && br.nr > 0 && nch > 0;
+    const bool some = b < v.nblocks && br.nr > 0 && nch > 0 && (LG == 6 || int64_t(br.nr) * nch <= p.large);
     const int gchan = some ? gptr(v.chan_map)[br.ch0] : -1;
     const bool mine = some && gchan >= 0 && gchan < p.nband;
     double fm = 0;
@@ -523,7 +564,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
         const int S = read_lane(pl.S, j), S2 = S * S;
 #pragma unroll
         for (int h = 0; h < H; ++h)
-          if (lane + 64 * h < S2) add(gc[h], wc[h]);
+          if (64 * h < S2) {  // (one branch a wavefront: without it the compiler selects, and adds all H every time)
+            if (lane + 64 * h < S2) add(gc[h], wc[h]);
+          }
         if (S2 > 64 * H) {
           const DDF_GLOBAL float2* cf = gptr(p.cf.data) + read_lane(pl.cfoff, j);
           const DDF_GLOBAL float2* q = grid + (read_lane(first, j) + int64_t(ip) * p.ny * p.nx);
@@ -541,7 +584,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
         }
       }
     }
-    if (!placed) continue;
+    if (!placed) return;
     M2 cv;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -592,7 +635,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
         st2(vp, make_float2(float(double(x0.x) - vb.a[0].re), float(double(x0.y) - vb.a[0].im)));
       }
     }
+  };
+  for (int64_t b0 = wave * NB; b0 < v.nblocks; b0 += nwaves * (LARGE ? kWave : NB)) {
+    if (LARGE) {
+      for (uint64_t take = large_blocks(p, b0, nwaves); take; take &= take - 1) block(b0 + __builtin_ctzll(take) * nwaves);
+    } else {
+      block(b0 + grp);
+    }
   }
+}
+
+// SPLIT: with the large blocks apart; held out where the map has none, for the registers (with Jones 119 spilled with,
+// 52 without).
+template <int NCORR, int JMODE, int LG, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(JMODE == 0 ? 4 : 3))) void degrid_plain(KParams p) {
+  if (SPLIT && blockIdx.x < p.large_wgs) {
+    const KParams& q = own_params();
+    degrid_part<NCORR, JMODE, 6, true>(q, plain_part<LG>(q, true));
+  } else degrid_part<NCORR, JMODE, LG, false>(p, plain_part<LG>(p, false));
 }
 
 // ---- BDA block index ---------------------------------------------------------------------------
@@ -841,13 +901,31 @@ int freq_means(const ddf_vis* v, double* fmean, double* wlmean, hipStream_t st) 
   return DDF_OK;
 }
 
-// Lanes of a block (log2: 0, 3 or 6): the mean visibilities per block of a map that covers the chunk, so
-// that a group's lanes have work; at least so many that the blocks give 4096 wavefronts.
+// Lanes of a block (log2: 0, 3 or 6), by the mean visibilities per block of a map that covers the chunk and by the
+// wavefronts that its blocks give.  Gridding / degridding with Jones of one facet, us with 1, 8 and 64 lanes (maps by
+// uvw, and of equal blocks):
+//   1 up to 10 visibilities, from 65536 blocks (1024 wavefronts): 287 000 blocks by uvw of 8 460 / 245, 475 / 278,
+//     1386 / 853; 386 000 of 13 862 / 415, 725 / 455, 1878 / 1178; 163 000 of 27 509 / 316, 439 / 296, 978 / 634;
+//     126 000 equal ones of 12 182 / 109, 217 / 143, 611 / 415; 25 000 of 4 86 / 71, 67 / 49, 144 / 121
+//   64 from 256: 165 000 by uvw of 54 -, 720 / 533, 1091 / 762; 56 000 equal ones of 160 -, 390 / 297, 559 / 488;
+//     11 000 of 320 -, 202 / 148, 178 / 132
+//   64 where 8 leave most of the GPU idle: 2100 blocks of 640 -, 271 / 201, 103 / 69; 1260 of 1 76 / 62, 34 / 33,
+//     31 / 32; 4200 of 24 -, 38 / 35, 54 / 46
 int plain_group(const ddf_vis* v) {
   const int64_t mean = v->nrow * v->nchan / std::max<int64_t>(1, v->nblocks);
-  const int64_t fill = int64_t(4096) * kWave / std::max<int64_t>(1, v->nblocks);
-  const int64_t lanes = std::max(mean, fill);
-  return lanes >= 48 ? 6 : lanes >= 4 ? 3 : 0;
+  if (mean <= 10 && v->nblocks >= 65536) return 0;
+  return mean >= 256 || v->nblocks < (mean >= 32 ? 4096 : 2048) ? 6 : 3;
+}
+// The large blocks of a map in a launch with 1 or 8 lanes a block: those of more than 32 turns of its lanes (8 lanes, 16
+// turns 1-20 % slower, 64 turns 5-25 %).  A group that took them itself was what the launch waited for: 18 700 blocks of
+// 26 visibilities on average (20 antennas close together), gridded and degridded with Jones 870 / 615 us by eights,
+// 224 / 171 by wavefronts, 170 / 135 with the large blocks apart.
+void plain_large(const ddf_vis* v, int lg, KParams& p) {
+  p.large = INT64_MAX;
+  p.large_wgs = 0;
+  if (lg == 6 || v->nblocks >= v->nrow * v->nchan) return;
+  p.large = int64_t(32) << lg;
+  p.large_wgs = unsigned(std::min<int64_t>(1024, (v->nblocks + 255) / 256));
 }
 unsigned grid_blocks(int64_t nblocks, int lg) {
   const int64_t per = 4 * (kWave >> lg);  // blocks of a workgroup
@@ -878,11 +956,17 @@ int launch_grid_r(const KParams& p, int jmode, int grid_f64, int lg, size_t lds,
   return launch_grid_t<READ, 0>(p, grid_f64, lg, lds, nb, st);
 }
 
+template <int NCORR, int JMODE, int LG>
+void launch_degrid_l(const KParams& p, unsigned nb, hipStream_t st) {
+  if (p.large_wgs) hipLaunchKernelGGL((degrid_plain<NCORR, JMODE, LG, true>), dim3(nb), dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((degrid_plain<NCORR, JMODE, LG, false>), dim3(nb), dim3(256), 0, st, p);
+}
+
 template <int NCORR, int JMODE>
 void launch_degrid_g(const KParams& p, int lg, unsigned nb, hipStream_t st) {
-  if (lg == 6) hipLaunchKernelGGL((degrid_plain<NCORR, JMODE, 6>), dim3(nb), dim3(256), 0, st, p);
-  else if (lg == 3) hipLaunchKernelGGL((degrid_plain<NCORR, JMODE, 3>), dim3(nb), dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((degrid_plain<NCORR, JMODE, 0>), dim3(nb), dim3(256), 0, st, p);
+  if (lg == 6) hipLaunchKernelGGL((degrid_plain<NCORR, JMODE, 6, false>), dim3(nb), dim3(256), 0, st, p);
+  else if (lg == 3) launch_degrid_l<NCORR, JMODE, 3>(p, nb, st);
+  else launch_degrid_l<NCORR, JMODE, 0>(p, nb, st);
 }
 
 template <int NCORR>
@@ -1028,7 +1112,8 @@ int ddf_grid(const ddf_grid_desc* g, const ddf_vis* v, const ddf_facet* f, void*
   size_t lds = (lds_base + (p.chan_lds ? 2 * size_t(v->nchan) : 0)) * 8;
   if (lds > 60 * 1024) return fail(DDF_EINVAL, "nband * npol too large for the gridding accumulators");
   const int lg = plain_group(v);
-  unsigned nb = grid_blocks(v->nblocks, lg);
+  plain_large(v, lg, p);
+  unsigned nb = grid_blocks(v->nblocks, lg) + p.large_wgs;
   if (sm.read == 4) rc = launch_grid_r<4>(p, jmode, g->grid_f64, lg, lds, nb, st);
   else if (sm.read == 2) rc = launch_grid_r<2>(p, jmode, g->grid_f64, lg, lds, nb, st);
   else rc = launch_grid_r<1>(p, jmode, g->grid_f64, lg, lds, nb, st);
@@ -1058,7 +1143,8 @@ int ddf_degrid(const ddf_grid_desc* g, const ddf_vis* v, const ddf_facet* f, voi
   fill_params(p, g, v, f, sm, starts, fmean0, wl_mean);
   const int jmode = f->jones.enabled ? f->jones.mode : 0;
   const int lg = plain_group(v);
-  unsigned nb = grid_blocks(v->nblocks, lg);
+  plain_large(v, lg, p);
+  unsigned nb = grid_blocks(v->nblocks, lg) + p.large_wgs;
   if (v->ncorr == 4) rc = launch_degrid_r<4>(p, jmode, lg, nb, st);
   else if (v->ncorr == 2) rc = launch_degrid_r<2>(p, jmode, lg, nb, st);
   else if (v->ncorr == 1) rc = launch_degrid_r<1>(p, jmode, lg, nb, st);
