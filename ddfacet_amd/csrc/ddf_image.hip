@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void facet_norm_kernel(const ImgFacet* F, int 
 // 32 pixels and turns each facet's tile over in LDS: both sides are read along their rows.  It first
 // lists the facets whose box meets its tile (a pixel has 3-4 of them, whatever their number) and takes
 // up to PL planes of one facet at a time, which share the taper, its inverse and SW.  121 facets of
-// 975^2, 4 bands: 2.4 ms; 16.3 with a lane per pixel testing every facet.
+// 975^2, 4 bands: 1.8 ms (2.4 in tiles of 32 x 32); 16.3 with a lane per pixel testing every facet.
 enum GatherMode { kStitch, kCutAdj };
 template <GatherMode MODE, int PL, int T>
 __global__ __launch_bounds__(256) void facet_gather(const ImgFacet* F, int nf, int n, int nband, int npol, int m,
@@ -625,7 +625,9 @@ int upload_facets(const ddf_image_facet* facets, int nf, int n, int m, hipStream
 
 // The centred transform of `nplanes` planes by the passes.  Columns of a strip: the most of 16, 8 and 4
 // that leave two workgroups a CU (80 KB of LDS each: 16 to 593 points, 8 to 1107, 4 to 1950); rows of a
-// workgroup: about 32 KB, at most 16.  Fewer rows where the launch would not give every CU two workgroups.
+// workgroup: about 32 KB, at most 16.  Fewer rows where the launch would not give every CU two workgroups: a
+// transform of one plane of 189^2 17-21 us, 26 with 16 rows; 36 of 525^2 123, 156 with a row (a line at 128 to 2048
+// workgroups is equal).
 int fft_planes(const FftDims& d, float2* planes, int64_t nplanes, int inverse, double scale, hipStream_t st) {
   const int n = d.n;
   const double norm = inverse ? scale : scale / (double(n) * double(n));
@@ -659,23 +661,22 @@ int fft_planes(const FftDims& d, float2* planes, int64_t nplanes, int inverse, d
 template <GatherMode MODE>
 int launch_gather(const ImgFacet* F, int nf, int n, int nband, int npol, int m, const float* norm, const int* use_norm,
                   float factor, int shift, float scale, float* image, hipStream_t st) {
-  // 32 x 32 pixels read 256-byte pieces of the facets; 16 x 16 where those would be fewer than two
-  // workgroups a CU (243^2 of 9 facets: 35 us with 32, 14 with 16)
+  // A plane alone: 16 x 16 pixels up to 1536 tiles of 32 x 32, which read longer pieces of the facets.  Stitch of
+  // 945^2 from 9 facets 93 us with 16, 98 with 32; 1575^2 of 25 223, 219; 3645^2 of 81 690, 654.  Planes together:
+  // 16 x 16, whose LDS lets more workgroups onto a CU: 243^2, 9 facets x 4 planes 88 us, 124 with 32; 6237^2, 121
+  // x 4 2.53 ms, 3.10.
   const unsigned groups = (unsigned(nband) * unsigned(npol) + 3) / 4, t32 = unsigned((m + 31) / 32), t16 = unsigned((m + 15) / 16);
-  const bool small = uint64_t(t32) * t32 * groups < 512, one = nband * npol == 1;
-  const unsigned tiles = small ? t16 : t32;
+  const bool one = nband * npol == 1, large = one && uint64_t(t32) * t32 > 1536;
+  const unsigned tiles = large ? t32 : t16;
   const dim3 g(tiles * groups, tiles), b(256);
-  if (one && small)
-    hipLaunchKernelGGL((facet_gather<MODE, 1, 16>), g, b, 0, st, F, nf, n, nband, npol, m, norm, use_norm, factor, shift,
-                       scale, image);
-  else if (one)
+  if (large)
     hipLaunchKernelGGL((facet_gather<MODE, 1, 32>), g, b, 0, st, F, nf, n, nband, npol, m, norm, use_norm, factor, shift,
                        scale, image);
-  else if (small)
-    hipLaunchKernelGGL((facet_gather<MODE, 4, 16>), g, b, 0, st, F, nf, n, nband, npol, m, norm, use_norm, factor, shift,
+  else if (one)
+    hipLaunchKernelGGL((facet_gather<MODE, 1, 16>), g, b, 0, st, F, nf, n, nband, npol, m, norm, use_norm, factor, shift,
                        scale, image);
   else
-    hipLaunchKernelGGL((facet_gather<MODE, 4, 32>), g, b, 0, st, F, nf, n, nband, npol, m, norm, use_norm, factor, shift,
+    hipLaunchKernelGGL((facet_gather<MODE, 4, 16>), g, b, 0, st, F, nf, n, nband, npol, m, norm, use_norm, factor, shift,
                        scale, image);
   HIP_OK(hipGetLastError());
   return DDF_OK;
