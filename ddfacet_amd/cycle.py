@@ -4,7 +4,7 @@ Device counterpart of the reference's per-chunk facet loop (ClassImagerDeconv.ma
 ClassFacetMachine.putChunkInBackground / FacetsToIm / getChunkInBackground,
 DDFacet/Imager/ClassDeconvMachine.py:1347-1395, ClassFacetMachine.py:912-1249, 1859-1943):
 
-    residual_image(vis)   grid every facet (batched plan), GridToIm (rocFFT, x OverS^2), stitch
+    residual_image(vis)   grid every facet (batched plan), GridToIm (centred inverse FFT, x OverS^2), stitch
                           with FacetNorm -> residual / dirty (or PSF) image on the main grid
     predict(model, vis)   GiveModelTessel + forward FFT per facet, then vis -= sum_f degrid_f
     cycle(model, vis)     predict then residual_image: one major cycle

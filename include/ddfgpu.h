@@ -225,14 +225,24 @@ int ddf_prepare_flags(uint8_t* flags, float* data, const int32_t* a0, const int3
  * model grid for degridding; facets[i].grid receives facet i's gridded visibilities.  All facets
  * share nw, overs, ref_wave, wmax and the per-plane supports (as ClassWTermModified builds them).
  * The Jones tables are taken from facets[0].jones; each facet supplies its direction indices and
- * its sum_jones / sum_jones_chan outputs.  vgrid / vdegrid carry the grid / degrid BDA maps.   */
+ * its sum_jones / sum_jones_chan outputs.  Gridding and the adjoint read the Jones time, channel and
+ * antenna maps at the call; degridding's runs of one Jones key are those of the maps when the plan was
+ * built, so a plan that degrids is rebuilt when they change (the tables themselves may change).
+ * vgrid / vdegrid carry the grid / degrid BDA maps.                                              */
 typedef struct ddf_plan ddf_plan;
 
 typedef struct ddf_plan_opts {
   int32_t tile;            /* uv tile edge in grid cells (0: 16)                                */
-  int32_t chunk;           /* max records per tile work item (0: 2048, fewer for small plans)    */
-  int32_t blocks_per_item; /* BDA blocks per gridding work item (0: 128)                        */
-  int32_t group;           /* facets per lane group in gridding (0: auto, <= 64)                */
+  int32_t chunk;           /* max records per tile work item (0: 2048, fewer for small plans; the
+                              adjoint 2048)                                                     */
+  int32_t blocks_per_item; /* BDA blocks per work item of grid pass A and of the adjoint's pass
+                              over the blocks (0: 128); without effect on gridding in the mixed
+                              precision with Jones by visibility, whose items are of about equal
+                              numbers of visibilities                                           */
+  int32_t group;           /* facets that a workgroup of grid pass A takes (0: auto, <= 64): lanes
+                              of a slot; with Jones by visibility in the mixed precision, facets
+                              that share the staged visibilities (0: as many as LDS holds the
+                              sums of)                                                          */
   int32_t precision;       /* 0 mixed: FP64 uvw rotation and per-row phase base, FP32 sin/cos and
                               FP32 phasor advance along channels (re-anchored every 16), FP32
                               run sums / Jones products / Stokes maps, FP64 stamp, facet and
